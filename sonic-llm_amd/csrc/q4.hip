@@ -434,11 +434,7 @@ __device__ __forceinline__ floatx4 scale_products(half4v a, u32x2 ws) {
 //
 // The kernel writes each slice's raw fp32 sums, part[slice][M][N]; whoever consumes them adds the slices in slice
 // order (k_q4_reduce here; the row kernels of the step), so the order of every sum is fixed by (N, K) alone.
-// FK (prompt rows, grid.y = 1): the workgroup walks every slice in turn, each summed into a fresh accumulator exactly
-// as its own launch would (the same groups, an odd slice's extra group added with scale 0 as its own ring pads it),
-// and adds the slices in slice order as the consumers do ((p0 + p1) + p2 ...), so part[0] holds, bit for bit, what
-// the consumers would have made of the split launch's slices: they read it as one slice.
-template <int WT, int MT, int S, bool FK, bool SW = false, bool GRP = false>
+template <int WT, int MT, int S, bool GRP>
 __device__ __forceinline__ void q4_gemm_ring(const GemmArgs& a) {
     constexpr int D = 2, FPW = MT;  // ring slots, fragments each wavefront stages
     // the loop below stages group i + 1 from register slot j (which holds group i's weights and group i + 1's records)
@@ -461,9 +457,7 @@ __device__ __forceinline__ void q4_gemm_ring(const GemmArgs& a) {
         mt0 = a.items[2 * blockIdx.z + 1];
     }
     mt0 = __builtin_amdgcn_readfirstlane(mt0);
-    // groups c0 .. c0 + ng - 1 (ng >= 1). FK: every group (the slices hold an even number of groups, so the walk is
-    // the groups in order, the last slice padded to an even count as its own launch pads it)
-    const int c0 = FK ? 0 : slice * a.gps, ng = FK ? a.ngroups : min(a.gps, a.ngroups - c0);
+    const int c0 = slice * a.gps, ng = min(a.gps, a.ngroups - c0);  // groups c0 .. c0 + ng - 1 (ng >= 1)
     const int s0 = set * (4 * S) + wave * S;
     const int sbytes = a.ngroups * TB;  // one stripe
     // one resource for the whole matrix, the wavefront's stripes by scalar offsets (stripes past the matrix read as
@@ -495,9 +489,9 @@ __device__ __forceinline__ void q4_gemm_ring(const GemmArgs& a) {
     u32x2 ws[D][S];
     u32x4 ra[D][FPW];
     float rk[D];
-    floatx4 acc[S][MT], tot[S][MT];
+    floatx4 acc[S][MT];
     for (int s = 0; s < S; ++s)
-        for (int mt = 0; mt < MT; ++mt) acc[s][mt] = tot[s][mt] = (floatx4){0.f, 0.f, 0.f, 0.f};
+        for (int mt = 0; mt < MT; ++mt) acc[s][mt] = (floatx4){0.f, 0.f, 0.f, 0.f};
 
     // a register slot holds the weights of group i and the activation records of group i + 1: the records are staged
     // into LDS an iteration before their group is summed, so loading them with the weights of the group before keeps
@@ -558,8 +552,6 @@ __device__ __forceinline__ void q4_gemm_ring(const GemmArgs& a) {
     }
     asm volatile("" ::"s"(a.part), "s"(a.N));  // (the tail's arguments read behind the first loads, as k_q4_gemm_s)
     const int trips = (ng + D - 1) / D;
-    int in_slice = 0;  // FK: groups of the current slice summed so far
-    bool first = true;
     for (int t = 0; t < trips; ++t)
         for (int j = 0; j < D; ++j) {
             const int i = t * D + j;
@@ -572,50 +564,9 @@ __device__ __forceinline__ void q4_gemm_ring(const GemmArgs& a) {
             // could not reuse the slot's scale registers, and the copy back at the loop's end waited on those loads
             for (int s = 0; s < S; ++s)
                 for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[s][mt]));
-            if constexpr (FK) {
-                if (++in_slice == a.gps || i == D * trips - 1) {  // the slice's last group: add the slice on
-                    in_slice = 0;
-                    for (int s = 0; s < S; ++s)
-                        for (int mt = 0; mt < MT; ++mt) {
-                            if (first) tot[s][mt] = acc[s][mt];
-                            else
-                                for (int v = 0; v < 4; ++v) tot[s][mt][v] = tot[s][mt][v] + acc[s][mt][v];
-                            acc[s][mt] = (floatx4){0.f, 0.f, 0.f, 0.f};
-                        }
-                    first = false;
-                }
-            }
             __builtin_amdgcn_sched_barrier(0);
             load(j, i + D);
         }
-    if constexpr (FK)
-        for (int s = 0; s < S; ++s)
-            for (int mt = 0; mt < MT; ++mt) acc[s][mt] = tot[s][mt];
-
-    if constexpr (SW) {
-        // SwiGLU of the tiles, as k_swiglu_quant makes it of the slices (the same sums: silu(gate) * up, Q8_0 blocks of
-        // 32 F columns): wavefront w's stripes are gate and up of F columns 64 set + 16 w .. + 15; the workgroup's 2 x 16
-        // rows x 64 columns go through LDS to threads (row, block of 32, lane part) for the quantizer
-        static_assert(FK && S == 2 && MT == 2, "the SwiGLU epilogue takes the FK walk with gate and up a wavefront");
-        __shared__ float s_h[32][64 + 4];
-        for (int mt = 0; mt < MT; ++mt)
-            for (int v = 0; v < 4; ++v) s_h[16 * mt + 4 * g + v][16 * wave + n_in] = silu(acc[0][mt][v]) * acc[1][mt][v];
-        __syncthreads();
-        const int t = threadIdx.x, r = t >> 3, blk = (t >> 2) & 1, gq = t & 3;
-        const int row = mt0 * 16 + r, F = a.N / 2, b = 2 * set + blk;
-        float v8[8];
-        for (int j = 0; j < 4; ++j) {
-            v8[j] = s_h[r][32 * blk + 4 * gq + j];
-            v8[4 + j] = s_h[r][32 * blk + 16 + 4 * gq + j];
-        }
-        if (row >= a.M || 32 * b >= F) return;  // (a block's 4 lane parts share the row and block: q8_store's shuffles)
-        float* o = a.h + (size_t) row * F + 32 * b;
-        *(float4*) (o + 4 * gq) = (float4){v8[0], v8[1], v8[2], v8[3]};
-        *(float4*) (o + 16 + 4 * gq) = (float4){v8[4], v8[5], v8[6], v8[7]};
-        q8_store(v8, gq, a.xo, F, row, b);
-        return;
-    }
-
     // lane (n, g) holds rows 4g + v of each row tile, column n of each of its stripes
     for (int s = 0; s < S; ++s) {
         const int stripe = s0 + s, col = stripe * 16 + n_in;
@@ -645,20 +596,11 @@ __device__ __forceinline__ void q4_gemm_ring(const GemmArgs& a) {
     else a.pos = pos_, a.seq = seq_
 #define GS_ARGS(a) (a).w, (a).xa, (a).M, (a).K, (a).nstripes, (a).ngroups, (a).gps, (a).pos, (a).seq, (a).N, (a).part, (a)
 #define GSG_ARGS(a) (a).w, (a).xa, (a).M, (a).K, (a).nstripes, (a).ngroups, (a).gps, (a).items, (a).count, (a).N, (a).part, (a)
-template <int WT, int MT, int S, bool FK = false, bool GRP = false>
+template <int WT, int MT, int S, bool GRP = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_q4_gemm(GS_PARAMS) {
     GS_TAKE();
-    q4_gemm_ring<WT, MT, S, FK, false, GRP>(a);
+    q4_gemm_ring<WT, MT, S, GRP>(a);
 }
-// the FK walk with two stripes a wavefront (prompt rows of the wide matrices): its accumulators and slice sums need
-// more than the 168 registers of 3 wavefronts a SIMD. SW: the gate|up matrix's SwiGLU + Q8_0 as its epilogue
-template <int WT, int MT, int S, bool SW = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_q4_gemm_fk2(GS_PARAMS) {
-    constexpr bool GRP = false;
-    GS_TAKE();
-    q4_gemm_ring<WT, MT, S, true, SW>(a);
-}
-
 // A k-slice sum of the workspace, read by the set's last workgroup from the XCD's L2, where the set's other
 // workgroups' stores are (the workgroup has dropped its L1 lines first: l1_drop)
 __device__ __forceinline__ float4 part_load4(__amdgpu_buffer_rsrc_t r, int off) {
@@ -1011,6 +953,231 @@ __global__ __launch_bounds__(256) void k_q4_gemm_s(GS_PARAMS) {
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// The matmul of many rows (prompts, large mixed steps): 32 x 32 x 16 MFMA tiles.
+//
+// A weight lane's dword of a Q4_0 block as signed fp16 integers: the nibbles taken by masks as fp16 subnormals
+// w 2^-24 (elements 4g..) and 16 w 2^-24 (16 + 4g..), then 8 (128) 2^-24 subtracted by packed fp16 adds, all exact: so
+// the block's MFMA needs no correction as its C input and gives isum 2^-24, every term a multiple of 2^-24 below 2^-1.
+// The fp32 sums are kept times 2^-24 (a power of two, so every fma rounds as the unscaled one) and multiplied back
+// when a slice is done. The masks are full-rate instructions here and the 1024 + w form's v_and_or and v_perm are
+// not (1.1 against 2 ns an instruction on a full SIMD).
+__device__ __forceinline__ half8 q4_signed(uint32_t w) {
+    const uint32_t h = w >> 8;  // (the tile keeps elements 0, 2, 1, 3 of a lane's four in bytes 0 .. 3)
+    const half8 v = __builtin_bit_cast(half8, (u32x4){w & 0x000F000Fu, h & 0x000F000Fu, w & 0x00F000F0u, h & 0x00F000F0u});
+    return v + __builtin_bit_cast(half8, (u32x4){0x80088008u, 0x80088008u, 0x80808080u, 0x80808080u});
+}
+#define Q4_SIGNED_SCALE 16777216.0f  // 2^24
+// The same of a Q8_0 block's two dwords: q and 16 q (the biased unpack less 1152 and 18432, exact)
+__device__ __forceinline__ half8 q8_signed(uint32_t w_lo, uint32_t w_hi) {
+    const _Float16 lo = 1152, hi = 18432;
+    return q8_unpack(w_lo, w_hi) - (half8){lo, lo, lo, lo, hi, hi, hi, hi};
+}
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx32 __attribute__((ext_vector_type(32)));
+
+// A wavefront holds MT tiles of 32 rows x 32 columns (two stripes); a workgroup WN of them side by side (32 MT rows x
+// 32 WN columns), times WK that walk different k-slices of the same tiles. Per group of 4 blocks the workgroup's
+// activation records go from global memory straight into one of two LDS buffers (each of the WK parts its own slice's)
+// while the group before is summed, and each wavefront's weights into one of two register sets; one barrier a group.
+// Per block and tile: two 32x32x16 MFMAs give the integer block sums, half a 32x32x4 two-block MFMA the products
+// dw * dx (A: dx one-hot over the 4 blocks, half the lanes a block; B: the tile's 4 scales as loaded), and 16 fmas.
+//
+// The order of the sums is the other kernels': each slice of the plan from zero, its groups in order, the slices added
+// in slice order. With WK > 1 a round of WK slices ends with the parts past the first handing their sums to the first
+// through LDS, which adds them one by one.
+//
+// What bounds it: per block and tile the MFMAs take 96 cycles and the wavefront's other 29 instructions 90, and the two
+// overlap little on this SIMD (32 MFMAs + 32 fmas took the sum of their times with 2 wavefronts a SIMD).
+//
+// Grid: 1-D, linear id L on XCD L mod 8. The XCDs are xm groups along the rows times 8 / xm along the columns, so that
+// an XCD's L2 holds its share of the activation: mx row tiles a group, interleaved.
+template <int WT, int MT, int WN, int WK, int OCC, bool SW>
+__global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(OCC, 8))) void k_q4_gemm_w(GS_PARAMS) {
+    constexpr bool GRP = false;
+    GS_TAKE();
+    constexpr bool Q8 = WT == WT_Q8_0;
+    constexpr int TB = Q8 ? Q8T_BYTES : Q4T_BYTES, SO = Q8 ? Q8T_SCALE_OFF : Q4T_SCALE_OFF;
+    constexpr int NW = Q8 ? 2 : 1;
+    constexpr int NF = MT * 8;  // fragments of a group's 2 MT row tiles of 16
+    __shared__ __attribute__((aligned(16))) uint8_t s_a0[WK][NF][1024], s_a1[WK][NF][1024];
+    __shared__ __attribute__((aligned(16))) float s_d0[WK][MT][2][64], s_d1[WK][MT][2][64];
+    __shared__ float s_x[WK > 1 ? WK - 1 : 1][WK > 1 ? WN : 1][WK > 1 ? MT * 16 : 1][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = WK > 1 ? wave % WN : wave, wk = WK > 1 ? wave / WN : 0;
+    const int r32 = lane & 31, h = lane >> 5;
+    const int mtiles = (a.M + 32 * MT - 1) / (32 * MT), xm = a.xm, mx = (mtiles + xm - 1) / xm;
+    const int xcd = blockIdx.x & 7, jb = blockIdx.x >> 3;
+    const int tile = (jb % mx) * xm + xcd % xm, set = (jb / mx) * (8 / xm) + xcd / xm;
+    if (tile >= mtiles || set * 2 * WN >= a.nstripes) return;
+    const int mt0 = tile * 2 * MT;  // the workgroup's first row tile of 16
+    const int s0 = (set * WN + wn) * 2;
+    const int sbytes = a.ngroups * TB, rstride = a.ngroups * XA_REC;
+    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(a.w, (uint32_t) (a.nstripes * sbytes));
+    const size_t x0 = (size_t) mt0 * rstride;
+    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(a.xa + x0, (uint32_t) (xa_bytes(a.M, a.K) - x0));
+    // lane (r32, h): MFMA j of a block takes the elements of lane part g = 2 j + h of both operands' tiles
+    const int w_off = (r32 >> 4) * sbytes + 16 * NW * ((r32 & 15) + 16 * h);
+    const int ws_off = (r32 >> 4) * sbytes + SO + 8 * (r32 & 15);
+    const int a_off = (r32 >> 4) * 4096 + 16 * ((r32 & 15) + 16 * h);
+    const int d_off = (r32 >> 4) * rstride + 64 * h + 4 * (r32 & 15);  // (pair p's block 2 p + h)
+
+    auto stage = [&](uint8_t (*sa)[1024], float (*sd)[2][64], int c) {
+        for (int j = 0; j < (NF + WN - 1) / WN; ++j) {
+            const int f = wn * ((NF + WN - 1) / WN) + j;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr) sa[f], 16, 16 * lane,
+                                                     (f / 4) * rstride + c * XA_REC + (f % 4) * 1024, 0, 0);
+        }
+        for (int k = wn; k < 2 * MT; k += WN)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr) sd[k / 2][k % 2], 4, d_off,
+                                                     (k / 2) * 2 * rstride + c * XA_REC + XA_DX_OFF + 128 * (k % 2), 0, 0);
+    };
+    struct W {
+        u32x4 q[2][NW];
+        u32x2 s;
+    };
+    auto wload = [&](W& w, int c) {
+        const int so = s0 * sbytes + c * TB;
+        for (int j = 0; j < 2; ++j)
+            for (int k = 0; k < NW; ++k) w.q[j][k] = bload16(wr, w_off + 512 * NW * j + 16 * k, so);
+        w.s = bload8(wr, ws_off, so);
+    };
+    floatx16 acc[MT], tot[MT];
+    for (int mt = 0; mt < MT; ++mt)
+        for (int v = 0; v < 16; ++v) acc[mt][v] = tot[mt][v] = 0.0f;
+    auto compute = [&](const uint8_t (*sa)[1024], const float (*sd)[2][64], const W& w) {
+        for (int p = 0; p < 2; ++p) {
+            half8 B[2][2];
+            for (int q = 0; q < 2; ++q)
+                for (int j = 0; j < 2; ++j) {
+                    const int b = 2 * p + q;
+                    if constexpr (Q8) B[q][j] = q8_signed(w.q[j][b / 2][2 * (b % 2)], w.q[j][b / 2][2 * (b % 2) + 1]);
+                    else B[q][j] = q4_signed(w.q[j][0][b]);
+                }
+            for (int mt = 0; mt < MT; ++mt) {
+                const uint32_t d = (uint32_t) __builtin_bit_cast(uint16_t, (_Float16) sd[mt][p][lane]) << (16 * h);
+                const half4v da = __builtin_bit_cast(half4v, p ? (u32x2){0u, d} : (u32x2){d, 0u});
+                floatx32 sc;
+                for (int v = 0; v < 32; ++v) sc[v] = 0.0f;
+                sc = __builtin_amdgcn_mfma_f32_32x32x4f16(da, __builtin_bit_cast(half4v, w.s), sc, 0, 0, 0);
+                for (int q = 0; q < 2; ++q) {
+                    const uint8_t* ap = &sa[0][0] + mt * 8192 + (2 * p + q) * 1024 + a_off;
+                    const half8 A0 = *(const half8*) ap, A1 = *(const half8*) (ap + 512);
+                    floatx16 is;
+                    for (int v = 0; v < 16; ++v) is[v] = 0.0f;
+                    is = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0, B[q][0], is, 0, 0, 0);
+                    is = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, B[q][1], is, 0, 0, 0);
+                    for (int v = 0; v < 16; ++v) acc[mt][v] = __builtin_fmaf(is[v], sc[16 * q + v], acc[mt][v]);
+                }
+            }
+        }
+    };
+    // the steps: rounds of WK slices, a round's steps those of its first (longest) slice; group(r, t) is the group that
+    // this part sums in step t of round r (past the part's slice: loaded, not summed)
+    const int gps = a.gps, rounds = (a.ks + WK - 1) / WK;
+    const int steps = (rounds - 1) * gps + min(gps, a.ngroups - (rounds - 1) * WK * gps);
+    int r = 0, t = 0;
+    auto group = [&](int rr, int tt) { return min((rr * WK + wk) * gps + tt, a.ngroups - 1); };
+    // a round's end: the slices' sums added on in slice order
+    auto fold = [&]() {
+        constexpr float US = Q8 ? 1.0f : Q4_SIGNED_SCALE;
+        if constexpr (WK > 1) {
+            if (wk > 0)
+                for (int mt = 0; mt < MT; ++mt)
+                    for (int v = 0; v < 16; ++v) s_x[wk - 1][wn][16 * mt + v][lane] = acc[mt][v] * US;
+            __syncthreads();
+        }
+        // (0 + the first slice's sum is that sum: a sum from zero is never -0; acc US is exact)
+        for (int mt = 0; mt < MT; ++mt)
+            for (int v = 0; v < 16; ++v) tot[mt][v] = __builtin_fmaf(acc[mt][v], US, tot[mt][v]), acc[mt][v] = 0.0f;
+        if constexpr (WK > 1) {
+            if (wk == 0)
+                for (int k = 1; k < WK; ++k)
+                    if (r * WK + k < a.ks)
+                        for (int mt = 0; mt < MT; ++mt)
+                            for (int v = 0; v < 16; ++v) tot[mt][v] += s_x[k - 1][wn][16 * mt + v][lane];
+        }
+        // (the next round's sums are written behind its groups' barriers, so behind these reads)
+    };
+    W w0, w1;
+    stage(s_a0[wk], s_d0[wk], group(0, 0));
+    wload(w0, group(0, 0));
+    auto step = [&](uint8_t (*sa)[1024], float (*sd)[2][64], W& w, uint8_t (*na)[1024], float (*nd)[2][64], W& nw) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wavefront's share of the group is staged, its weights here
+        __syncthreads();
+        const bool end = t + 1 == gps;
+        const int ng = end ? group(r + 1, 0) : group(r, t + 1);
+        stage(na, nd, ng);
+        wload(nw, ng);
+        __builtin_amdgcn_sched_barrier(0);
+        if (WK == 1 || (r * WK + wk) * gps + t < a.ngroups) compute(sa, sd, w);
+        ++t;
+        if (end) {
+            fold();
+            ++r, t = 0;
+        }
+    };
+    for (int i = 0; i < steps; i += 2) {
+        step(s_a0[wk], s_d0[wk], w0, s_a1[wk], s_d1[wk], w1);
+        if (i + 1 < steps) step(s_a1[wk], s_d1[wk], w1, s_a0[wk], s_d0[wk], w0);
+    }
+    if (t > 0) fold();  // (a last round of fewer steps)
+    // lane (r32, h): column r32 of the wavefront's 32, rows 8 (v / 4) + 4 h + v % 4 of each tile
+    // (the lane's numbers formed again, so that no register holds them through the walk)
+    const int row0 = mt0 * 16, el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const int er = el & 31, eh = el >> 5;
+    if constexpr (SW) {
+        // SwiGLU: the wavefront's two stripes are gate and up of 16 F columns (lanes r32 and r32 + 16); the workgroup's
+        // rows x 16 WN F columns go through LDS to threads (row, Q8_0 block, lane part) for the quantizer
+        constexpr int HC = 16 * WN, HW = HC + 4;
+        __shared__ float s_h[32 * MT][HW];
+        if (wk == 0)
+            for (int mt = 0; mt < MT; ++mt)
+                for (int v = 0; v < 16; ++v) {
+                    const float u = __shfl_xor(tot[mt][v], 16);
+                    if (er < 16) s_h[32 * mt + 8 * (v / 4) + 4 * eh + v % 4][16 * wn + er] = silu(tot[mt][v]) * u;
+                }
+        __syncthreads();
+        const int F = a.N / 2;
+        for (int it = 64 * wave + el; it < 32 * MT * (HC / 32) * 4; it += 64 * WN * WK) {
+            const int gq = it & 3, blk = (it >> 2) % (HC / 32), rr = (it >> 2) / (HC / 32);
+            const int row = row0 + rr, b = set * (HC / 32) + blk;
+            float v8[8];
+            for (int j = 0; j < 4; ++j) {
+                v8[j] = s_h[rr][32 * blk + 4 * gq + j];
+                v8[4 + j] = s_h[rr][32 * blk + 16 + 4 * gq + j];
+            }
+            if (row >= a.M || 32 * b >= F) continue;  // (a block's 4 lane parts together: q8_store's shuffles)
+            float* o = a.h + (size_t) row * a.ldy + 32 * b;
+            const bool whole = 32 * b + 32 <= F;  // (F a multiple of 16)
+            if (a.vec) {
+                *(float4*) (o + 4 * gq) = (float4){v8[0], v8[1], v8[2], v8[3]};
+                if (whole) *(float4*) (o + 16 + 4 * gq) = (float4){v8[4], v8[5], v8[6], v8[7]};
+            } else {
+                for (int j = 0; j < 4; ++j) {
+                    o[4 * gq + j] = v8[j];
+                    if (whole) o[16 + 4 * gq + j] = v8[4 + j];
+                }
+            }
+            if (a.xo) q8_store(v8, gq, a.xo, F, row, b);
+        }
+        return;
+    }
+    const int col = s0 * 16 + er;
+    if (wk > 0 || col >= a.N) return;
+    float* o = a.y + (size_t) row0 * a.ldy + col;
+    const int nr = a.M - row0;
+    for (int mt = 0; mt < MT; ++mt)
+        for (int v = 0; v < 16; ++v) {
+            const int rr = 32 * mt + 8 * (v / 4) + 4 * eh + v % 4;
+            if (rr < nr) {
+                if (a.epi == EPI_ADD) o[(size_t) rr * a.ldy] += tot[mt][v];
+                else o[(size_t) rr * a.ldy] = tot[mt][v];
+            }
+        }
+}
+
 // The few-row matmul (M <= 4 rows: the reference's mat-vec rows, mv_q4, kernels.metal:1324-1411). One lane per output
 // column: a wavefront takes 4 stripes (64 columns), a workgroup 16, and the plan's k-slices go across workgroups as
 // the MFMA kernels split them. The slice's activation rows are staged once into LDS as int8 (from the operand's fp16
@@ -1158,7 +1325,7 @@ __global__ void k_q4_reduce(GemmArgs a) {
 // round of loads per workgroup) beat fewer, longer workgroups for the layer-sized matrices, while every slice costs
 // the consumer one more partial sum to read.
 #define Q4_WIDE (8 * 768)  // stripes of an LM-head-wide matrix
-#define Q4_PAIR_ROWS 256   // rows from which every matrix takes its row tiles in pairs
+#define Q4_MANY_ROWS 256   // rows from which every matrix takes the many-row kernel
 GemmPlan q4_plan(int N, int K, int wt) {
     GemmPlan p;
     p.nstripes = (N + 15) / 16;
@@ -1201,7 +1368,7 @@ GemmPlan q4_plan(int N, int K, int wt) {
     // step against depth 2, A/B in one call: decode 8,274 -> 8,281 tok/s, Qwen3-30B-A3B 4,827 -> 4,862; depth 4 for
     // the gate|up matrix as well cost decode 0.45%, for q|k|v 0.6% and for down 0.7%
     p.sd = wt == WT_Q4_0 && narrow_deep && p.sspw == 1 ? 4 : 2;
-    // the ring kernel (prompt rows) with the same slices: one stripe a wavefront
+    // the ring kernel (slices of more than 8 groups): one stripe a wavefront
     p.spw = 1;
     p.sets = (p.nstripes + 3) / 4;
     return p;
@@ -1209,21 +1376,20 @@ GemmPlan q4_plan(int N, int K, int wt) {
 
 size_t q4_workspace_bytes(int M, int N, int K, int wt) { return (size_t) q4_plan(N, K, wt).ks * M * N * sizeof(float); }
 
-// (FK: one stripe a wavefront only, the plan of every split layer matrix)
-template <int WT, bool FK = false>
+template <int WT>
 static void launch_gemm(int mt, int spw, dim3 grid, const GemmArgs& a, hipStream_t st) {
-    if constexpr (WT == WT_Q4_0 && !FK) {
+    if constexpr (WT == WT_Q4_0) {
         if (mt == 1) {
-            if (spw == 2) hipLaunchKernelGGL((k_q4_gemm<WT, 1, 2, FK>), grid, dim3(256), 0, st, GS_ARGS(a));
-            else hipLaunchKernelGGL((k_q4_gemm<WT, 1, 1, FK>), grid, dim3(256), 0, st, GS_ARGS(a));
+            if (spw == 2) hipLaunchKernelGGL((k_q4_gemm<WT, 1, 2>), grid, dim3(256), 0, st, GS_ARGS(a));
+            else hipLaunchKernelGGL((k_q4_gemm<WT, 1, 1>), grid, dim3(256), 0, st, GS_ARGS(a));
         } else {
-            if (spw == 2) hipLaunchKernelGGL((k_q4_gemm<WT, 2, 2, FK>), grid, dim3(256), 0, st, GS_ARGS(a));
-            else hipLaunchKernelGGL((k_q4_gemm<WT, 2, 1, FK>), grid, dim3(256), 0, st, GS_ARGS(a));
+            if (spw == 2) hipLaunchKernelGGL((k_q4_gemm<WT, 2, 2>), grid, dim3(256), 0, st, GS_ARGS(a));
+            else hipLaunchKernelGGL((k_q4_gemm<WT, 2, 1>), grid, dim3(256), 0, st, GS_ARGS(a));
         }
-    } else {  // Q8_0: one stripe per wavefront (q4_plan); FK likewise
+    } else {  // Q8_0: one stripe per wavefront (q4_plan)
         (void) spw;
-        if (mt == 1) hipLaunchKernelGGL((k_q4_gemm<WT, 1, 1, FK>), grid, dim3(256), 0, st, GS_ARGS(a));
-        else hipLaunchKernelGGL((k_q4_gemm<WT, 2, 1, FK>), grid, dim3(256), 0, st, GS_ARGS(a));
+        if (mt == 1) hipLaunchKernelGGL((k_q4_gemm<WT, 1, 1>), grid, dim3(256), 0, st, GS_ARGS(a));
+        else hipLaunchKernelGGL((k_q4_gemm<WT, 2, 1>), grid, dim3(256), 0, st, GS_ARGS(a));
     }
 }
 
@@ -1255,19 +1421,72 @@ static bool launch_gemv(const GemmPlan& p, const GemmArgs& a, hipStream_t st) {
     return true;
 }
 
+// Whether a matmul of M rows takes the many-row kernel (k_q4_gemm_w): every one from 256 rows on; below that where the
+// other kernels' slices cost more than the wide tiles leave idle, T tiles of 32 x 32 in all. Measured on MI355X, Q4_0,
+// the streaming kernel with its slice sum against this one (us): 19456 x 2560 at 100 rows (T = 2432) 32.6 / 26.3, at
+// 64 (1216) 21.9 / 20.8; 2560 x 4096 at 192 rows (480) 18.2 / 15.1; 2560 x 9728 at 192 (480) 28.5 / 31.4.
+static bool wide_takes(int M, const GemmPlan& p) {
+    const long T = (long) ((M + 31) / 32) * ((p.nstripes + 1) / 2);
+    return M >= Q4_MANY_ROWS || (M >= 96 && T >= 2048) || (M >= 192 && p.ngroups <= 32);
+}
+static GemmArgs wide_args(const uint8_t* w, const uint8_t* xa, int M, int N, int K, const GemmPlan& p) {
+    GemmArgs a{};
+    a.w = w; a.xa = xa;
+    a.M = M; a.N = N; a.K = K; a.epi = EPI_STORE;
+    a.nstripes = p.nstripes; a.ngroups = p.ngroups; a.ks = p.ks; a.gps = p.gps;
+    return a;
+}
+template <int WT, int MT, int WN, int WK, int OCC, bool SW>
+static void launch_w(const GemmPlan& p, GemmArgs& a, hipStream_t st) {
+    const int mts = (a.M + 32 * MT - 1) / (32 * MT), sets = (p.nstripes + 2 * WN - 1) / (2 * WN);
+    // the XCDs split the rows while an XCD's share of the activation is over half its 4 MB L2 (each then reads every
+    // weight, the smaller traffic: 2048 rows of 19456 x 2560, 266 us with 8 row groups, 288 with 1) and no more than
+    // 1/16 of the row tiles are padding
+    const long abytes = (long) xa_bytes(a.M, a.K);
+    int xm = 1;
+    while (xm < 8 && abytes / xm > (2 << 20) && 16 * ((mts + 2 * xm - 1) / (2 * xm) * 2 * xm) <= 17 * mts) xm *= 2;
+    a.xm = xm;
+    const dim3 grid(8 * ((mts + xm - 1) / xm) * ((sets + 8 / xm - 1) / (8 / xm)));
+    hipLaunchKernelGGL((k_q4_gemm_w<WT, MT, WN, WK, OCC, SW>), grid, dim3(64 * WN * WK), 0, st, GS_ARGS(a));
+}
+// The launch's tiles, by T_64 (T_32) = the 32 x 32 tiles with the rows padded to 64 (32), us on MI355X as (two row tiles
+// a wavefront; one; one and two k-slices at a time): 19456 x 2560 at 512 rows, T = 9728: 73 78 95; 6144 x 2560 at 1024,
+// 6144: 47 50 63; at 512, 3072: 33 28 34; 2560 x 9728 at 768, 1920: 86 67 73; at 512, 1280: 86 66 53. Two row tiles
+// unpack a weight once for both, but need 168 registers (Q8_0's would spill); fewer than 2 tiles a SIMD leave it idle
+// unless the slices are split too.
+static void launch_wide(int wt, bool sw, const GemmPlan& p, GemmArgs& a, hipStream_t st) {
+    const long nt = (p.nstripes + 1) / 2, t32 = (long) ((a.M + 31) / 32) * nt, t64 = (long) ((a.M + 63) / 64) * 2 * nt;
+    const int cfg = t32 < 1800 && p.ks > 1 ? 2 : wt == WT_Q4_0 && t32 >= 6000 && 15 * t64 <= 16 * t32 ? 0 : 1;
+    if (wt == WT_Q8_0) {
+        if (cfg == 2) sw ? launch_w<WT_Q8_0, 1, 2, 2, 3, true>(p, a, st) : launch_w<WT_Q8_0, 1, 2, 2, 3, false>(p, a, st);
+        else sw ? launch_w<WT_Q8_0, 1, 4, 1, 3, true>(p, a, st) : launch_w<WT_Q8_0, 1, 4, 1, 3, false>(p, a, st);
+    } else {
+        if (cfg == 2) sw ? launch_w<WT_Q4_0, 1, 2, 2, 3, true>(p, a, st) : launch_w<WT_Q4_0, 1, 2, 2, 3, false>(p, a, st);
+        else if (cfg == 1) sw ? launch_w<WT_Q4_0, 1, 4, 1, 3, true>(p, a, st) : launch_w<WT_Q4_0, 1, 4, 1, 3, false>(p, a, st);
+        else sw ? launch_w<WT_Q4_0, 2, 4, 1, 3, true>(p, a, st) : launch_w<WT_Q4_0, 2, 4, 1, 3, false>(p, a, st);
+    }
+}
+
 int q4_gemm_raw(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* part, size_t part_bytes,
                 hipStream_t st, int wt) {
     if (M <= 0) return 0;
     if (wt != WT_Q4_0 && wt != WT_Q8_0) return -1;
     const GemmPlan p = q4_plan(N, K, wt);
     if (part == nullptr || part_bytes < (size_t) p.ks * M * N * sizeof(float)) return -1;
+    if (wide_takes(M, p)) {  // the slices' sum itself, as one slice
+        GemmArgs a = wide_args(w, xa, M, N, K, p);
+        a.y = part;
+        a.ldy = N;
+        launch_wide(wt, false, p, a, st);
+        return 1;
+    }
     GemmArgs a{};
     a.w = w; a.xa = xa; a.part = part; a.y = nullptr;
     a.M = M; a.N = N; a.K = K; a.ldy = 0; a.epi = EPI_STORE;
     a.nstripes = p.nstripes; a.ngroups = p.ngroups; a.ks = p.ks; a.gps = p.gps;
     a.mtiles = (M + 15) / 16;
     if (wt == WT_Q4_0 && M <= GEMV_ROWS && launch_gemv(p, a, st)) return p.ks;  // few rows: the per-column GEMV
-    if (p.stream && a.M < Q4_PAIR_ROWS) {  // the streaming kernel (ring depth 2)
+    if (p.stream) {  // the streaming kernel
         const int mt = std::min(p.smt, a.mtiles);
         const dim3 grid((p.nstripes + 4 * p.sspw - 1) / (4 * p.sspw), p.ks, (a.mtiles + mt - 1) / mt);
         const bool ok = wt == WT_Q8_0 ? launch_gemm_s<WT_Q8_0>(mt, p.sspw, 2, p.gps, grid, a, st)
@@ -1277,31 +1496,8 @@ int q4_gemm_raw(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float*
     // row tiles of 16 per workgroup (grid z: one per tile) for matrices narrower than 512 stripes: twice the workgroups
     // and loads in flight (q|k|v, o, down: 8.4 against 9.1 us at 32 rows; the two workgroups of a tile pair run on the
     // same XCD, so the second reads the weights from its L2); pairs of tiles for the wider ones (the Q8_0 gate|up and
-    // the LM heads were slower with single tiles, the Q4_0 gate|up the same), and for every matrix from Q4_PAIR_ROWS
-    // rows on (prompt rows; Qwen3-4B at 512 rows a step: 15.9 ms a step against 16.3 with the narrow ones single and
-    // 16.6 all single; 4 tiles, at 2 wavefronts a SIMD for their registers, 17.5). Either way a row's sums are the same
-    // (same slices, same order).
-    const int mt = a.mtiles == 1 || (p.nstripes < 512 && a.M < Q4_PAIR_ROWS) ? 1 : 2;
-    // prompt rows: one workgroup walks every slice of its tiles and leaves their sum in part[0] (the same bits the
-    // consumers make of the slices), so no slice is written or read back (at 512 rows the split launches wrote 16-120
-    // MB of slices a matrix)
-    if (a.M >= Q4_PAIR_ROWS && p.ks > 1 && p.spw == 1 && p.gps % 2 == 0) {
-        // Qwen3-4B at 512 rows a step (launches of one sequence's prompt): 2 stripes a wavefront for the wide q|k|v
-        // and gate|up (33 and 92 us against 42 and 119 with one; 4 stripes: 42 and 92), one for o and down (54 us
-        // against 60 with two); 40.7k -> 43.3k prompt tok/s on one box. The split launches and their slices: 34.7k.
-        // o and down (fewer than 384 stripes) in single row tiles: twice their workgroups, 45.0k against 44.1k tok/s
-        // with tile pairs (q|k|v in single tiles: 44.5k)
-        const int fmt = p.nstripes < 384 ? 1 : 2;
-        if (wt == WT_Q4_0 && p.nstripes >= 384) {
-            const dim3 grid((p.nstripes + 7) / 8, 1, (a.mtiles + 1) / 2);
-            hipLaunchKernelGGL((k_q4_gemm_fk2<WT_Q4_0, 2, 2>), grid, dim3(256), 0, st, GS_ARGS(a));
-        } else {
-            const dim3 grid(p.sets, 1, (a.mtiles + fmt - 1) / fmt);
-            if (wt == WT_Q8_0) launch_gemm<WT_Q8_0, true>(fmt, 1, grid, a, st);
-            else launch_gemm<WT_Q4_0, true>(fmt, 1, grid, a, st);
-        }
-        return 1;
-    }
+    // the LM heads were slower with single tiles). Either way a row's sums are the same (same slices, same order).
+    const int mt = a.mtiles == 1 || p.nstripes < 512 ? 1 : 2;
     const dim3 grid(p.sets, p.ks, mt == 1 ? a.mtiles : (a.mtiles + 1) / 2);
     if (wt == WT_Q8_0) launch_gemm<WT_Q8_0>(mt, p.spw, grid, a, st);
     else launch_gemm<WT_Q4_0>(mt, p.spw, grid, a, st);
@@ -1329,7 +1525,7 @@ static bool launch_gemm_fe(int mt, int spw, int gps, dim3 grid, const GemmArgs& 
 // nxcd); false when the plan, the weight type or the epilogue's unit does not allow one
 static bool fused_shape(int M, int N, int K, int wt, int fe, int nxcd, int cnt_len, GemmPlan& p, int& spw, int& mt,
                         dim3& grid) {
-    if (M <= 0 || M >= Q4_PAIR_ROWS || nxcd < 1 || (wt != WT_Q4_0 && wt != WT_Q8_0)) return false;
+    if (M <= 0 || M >= Q4_MANY_ROWS || nxcd < 1 || (wt != WT_Q4_0 && wt != WT_Q8_0)) return false;
     p = q4_plan(N, K, wt);
     if (!p.stream || p.gps > 8) return false;
     // a set must hold whole epilogue units: one head (8 stripes: two a wavefront, Q4_0 tiles), or S Q8_0 blocks of
@@ -1506,10 +1702,10 @@ int q4_gemm_grouped(const uint8_t* w, size_t wstride, const int32_t* items, cons
     // (K past 16 groups) the ring kernel. Q4_0: 2 stripes a wavefront; Q8_0 tiles take one (twice the weight
     // registers)
     if (wt == WT_Q8_0) {
-        hipLaunchKernelGGL((k_q4_gemm<WT_Q8_0, 1, 1, false, true>), dim3((a.nstripes + 3) / 4, 1, max_items), dim3(256), 0,
+        hipLaunchKernelGGL((k_q4_gemm<WT_Q8_0, 1, 1, true>), dim3((a.nstripes + 3) / 4, 1, max_items), dim3(256), 0,
                            st, GSG_ARGS(a));
     } else {
-        hipLaunchKernelGGL((k_q4_gemm<WT_Q4_0, 1, 2, false, true>), dim3((a.nstripes + 7) / 8, 1, max_items), dim3(256), 0,
+        hipLaunchKernelGGL((k_q4_gemm<WT_Q4_0, 1, 2, true>), dim3((a.nstripes + 7) / 8, 1, max_items), dim3(256), 0,
                            st, GSG_ARGS(a));
     }
     return 1;
@@ -1539,9 +1735,9 @@ int q4_gemm_grouped_swiglu(const uint8_t* w, size_t wstride, const int32_t* item
 }
 
 bool q4_gemm_swiglu_fits(int M, int N, int K, int wt) {
-    if (wt != WT_Q4_0 || M < Q4_PAIR_ROWS || N % 256 != 0) return false;
+    if (wt != WT_Q4_0 || M < Q4_MANY_ROWS || N % 256 != 0) return false;
     const GemmPlan p = q4_plan(N, K, wt);
-    return p.ks > 1 && p.spw == 1 && p.gps % 2 == 0 && p.nstripes >= 384;  // (the FK walk's shapes)
+    return p.ks > 1 && p.spw == 1 && p.gps % 2 == 0 && p.nstripes >= 384;
 }
 
 int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* h, uint8_t* xo, hipStream_t st,
@@ -1553,8 +1749,9 @@ int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, flo
     a.M = M; a.N = N; a.K = K; a.epi = EPI_STORE;
     a.nstripes = p.nstripes; a.ngroups = p.ngroups; a.ks = p.ks; a.gps = p.gps;
     a.mtiles = (M + 15) / 16;
-    const dim3 grid((p.nstripes + 7) / 8, 1, (a.mtiles + 1) / 2);
-    hipLaunchKernelGGL((k_q4_gemm_fk2<WT_Q4_0, 2, 2, true>), grid, dim3(256), 0, st, GS_ARGS(a));
+    a.ldy = N / 2;
+    a.vec = 1;
+    launch_wide(wt, true, p, a, st);
     return 1;
 }
 
@@ -1568,6 +1765,17 @@ void q4_reduce_slices(const float* part, int ks, int M, int N, float* y, hipStre
 int q4_gemm(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* y, int ldy, int epi, float* ws,
             size_t ws_bytes, hipStream_t st, int wt) {
     if (M <= 0) return 0;
+    if (wt != WT_Q4_0 && wt != WT_Q8_0) return -1;
+    const GemmPlan p = q4_plan(N, K, wt);
+    if (wide_takes(M, p)) {  // the many-row kernel applies the epilogue itself (the workspace is asked for, not used)
+        if (ws == nullptr || ws_bytes < (size_t) p.ks * M * N * sizeof(float)) return -1;
+        GemmArgs a = wide_args(w, xa, M, N, K, p);
+        a.y = a.h = y;
+        a.ldy = ldy; a.epi = epi;
+        a.vec = ldy % 4 == 0 && (uintptr_t) y % 16 == 0;
+        launch_wide(wt, epi == EPI_SWIGLU, p, a, st);
+        return 0;
+    }
     const int ks = q4_gemm_raw(w, xa, M, N, K, ws, ws_bytes, st, wt);
     if (ks < 0) return -1;
     GemmArgs a{};
@@ -1673,7 +1881,7 @@ int resid_quant(float* x, const float* part, int ks, int M, int K, const float* 
     // where that matmul streams its slices)
     WeightPrefetch pf{};
     int npf = 0;
-    if (next_w && M < Q4_PAIR_ROWS) {
+    if (next_w && M < Q4_MANY_ROWS) {
         const GemmPlan p = q4_plan(next_N, next_K, wt);
         const int tb = wt_tile_bytes(wt);
         if (p.stream) {

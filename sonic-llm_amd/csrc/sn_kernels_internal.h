@@ -46,6 +46,8 @@ struct GemmArgs {
     uint16_t *kpool, *vpool;
     int H, KVH;
     const float2* rope_cs;  // the rows' rotation table (rope_table), or null (each head forms its angles)
+    // (k_q4_gemm_w) the XCD groups along the rows; whether h takes 16-byte stores (its rows ldy apart)
+    int xm, vec;
 };
 // the streaming kernel's fused epilogues: none (the k-slice sums for the row kernels), the SwiGLU + Q8_0 of a
 // stripe-interleaved gate|up matrix (k_swiglu_quant's arithmetic), the q|k|v heads' QK-norm + RoPE + cache write
@@ -79,8 +81,8 @@ GemmPlan q4_plan(int N, int K, int wt = WT_Q4_0);
 // the raw matmul with an explicit plan (tuning): mt row tiles a workgroup, spw stripes a wavefront, G groups a slice
 // loaded at once (G 0: the default plan); the slice count, or -1
 // part[ks][M][N] added in slice order into y [M][N]
-// The prompt rows' gate|up matmul with its SwiGLU: from Q4_PAIR_ROWS rows, a Q4_0 stripe-interleaved matrix of
-// N = 2F (F a multiple of 128) walked whole (k_q4_gemm_w2, FK) with silu(gate) * up written as fp32 rows h [M][F] and
+// The prompt rows' gate|up matmul with its SwiGLU: from 256 rows, a Q4_0 stripe-interleaved matrix of N = 2F (F a
+// multiple of 128) through the many-row kernel (k_q4_gemm_w) with silu(gate) * up written as fp32 rows h [M][F] and
 // as the Q8_0 operand xo (K = F), the same bits as the matmul's slices through k_swiglu_quant. xo must not be xa.
 // Returns 1, or 0 when the shape does not qualify (nothing launched: use the matmul and swiglu_quant).
 int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* h, uint8_t* xo, hipStream_t st,

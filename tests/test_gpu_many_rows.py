@@ -1,0 +1,71 @@
+"""The many-row matmul (k_q4_gemm_w) against the few-row kernels, bit for bit: a row's sums depend on the row alone, so
+M rows in one call equal the same rows in calls of 16 (which tests/test_gpu_q4.py and test_gpu_q8.py hold to the oracle).
+Sizes at the edges of its tiles (32 rows, 64 with two row tiles a wavefront; 128 or 64 columns a workgroup), of its
+launch choices and of the k-slices (short last slices, an odd number of slices taken two at a time), ragged N and K."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch  # noqa: F401 (its HIP runtime is the process's: loaded before the library)
+
+import sllm_next as S
+from tests import gpu_util as U
+
+pytestmark = pytest.mark.gpu
+STORE, ADD, SWIGLU = 0, 1, 2
+
+
+def weights(r, N, K, wt):
+    f = S.quantize_q4_0 if wt == 2 else None
+    x = (r.standard_normal((N, K)) * 0.02).astype(np.float32)
+    if wt == 2:
+        return f(x)
+    out = np.empty(N * (K // 32) * 34, np.uint8)
+    S.lib().snx_quantize_q8_0(S._p(x), S._p(out), x.size)
+    return out
+
+
+def matmul(L, wt, w, x, N, epi, ldy, y0, off=0):
+    """y0 with the product of rows x written (or added) at element offset `off` of a larger buffer"""
+    M, K = x.shape
+    xa, y = U.empty(L.snk_xa_bytes(M, K)), U.dev(y0)
+    assert L.snk_quant_act(U.ptr(U.dev(x)), M, K, K, None, 1e-6, U.ptr(xa), U.stream()) == 0
+    nb = (L.snk_q4_workspace_bytes if wt == 2 else L.snk_q8_workspace_bytes)(M, N, K)
+    ws = U.empty(nb)
+    f = L.snk_q4_gemm if wt == 2 else L.snk_q8_gemm
+    assert f(U.ptr(w), U.ptr(xa), M, N, K, C.c_void_p(y.data_ptr() + 4 * off), ldy, epi, U.ptr(ws), nb, U.stream()) == 0
+    return U.host(y, np.float32, y0.shape)
+
+
+CASES = [  # wt, M, N, K, epi, ldy - columns, offset of y in floats
+    (2, 256, 1000, 4096, STORE, 0, 0),      # two slices at a time; ragged columns
+    (2, 257, 2560, 1280, ADD, 3, 1),        # 3 slices of 4 groups, one row past the tiles, y unaligned
+    (2, 333, 2576, 9728 // 2, STORE, 5, 0),  # a short last slice
+    (2, 192, 6144, 2560, STORE, 0, 0),      # below 256 rows
+    (2, 100, 19456, 1056, SWIGLU, 0, 0),    # wide at 100 rows; K not a multiple of 128
+    (2, 384, 19456, 1024, SWIGLU, 0, 0),    # two row tiles a wavefront, one slice
+    (2, 512, 12320, 2080, ADD, 0, 2),       # two row tiles, ragged columns and K, y off 16 bytes
+    (2, 260, 1056, 2048, SWIGLU, 1, 0),     # F a multiple of 16 alone, rows of h unaligned
+    (8, 256, 1040, 2560, STORE, 0, 0),      # Q8_0: two slices at a time
+    (8, 300, 6160, 1280, ADD, 0, 0),        # Q8_0: one slice at a time
+    (8, 200, 4096, 1024, SWIGLU, 4, 0),
+]
+
+
+@pytest.mark.parametrize("wt,M,N,K,epi,pad,off", CASES)
+def test_many_rows_are_the_few_rows_bits(wt, M, N, K, epi, pad, off):
+    L, r = S.lib(), np.random.default_rng(M * 7 + N)
+    raw = U.dev(weights(r, N, K, wt))
+    w = U.empty((L.snk_q4_stripes_bytes if wt == 2 else L.snk_q8_tiles_bytes)(N, K))
+    assert (L.snk_q4_repack if wt == 2 else L.snk_q8_repack)(U.ptr(raw), N, K, U.ptr(w), U.stream()) == 0
+    x = r.standard_normal((M, K)).astype(np.float32)
+    cols = N // 2 if epi == SWIGLU else N
+    ldy = cols + pad
+    y0 = r.standard_normal(M * ldy + off + 8).astype(np.float32)
+    want = y0.copy()
+    for m in range(0, M, 16):
+        n = min(16, M - m)
+        part = want[off + m * ldy:off + m * ldy + n * ldy].copy()
+        want[off + m * ldy:off + m * ldy + n * ldy] = matmul(L, wt, w, x[m:m + n], N, epi, ldy, part)
+    got = matmul(L, wt, w, x, N, epi, ldy, y0, off)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
