@@ -93,7 +93,19 @@ __device__ __forceinline__ float block_reduce_sum256(float v, float* red) {
     return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__device__ __forceinline__ void q8_store(const float* v, int g, uint8_t* xa, int K, int m, int b);
+// thread t's part of a row's sum of squares (elements t, t + 256, ..., in order; 8 loads in flight)
+__device__ __forceinline__ float row_squares(const float* x, int K, int t) {
+    float s = 0.0f;
+    for (int i = t; i < K; i += 256 * 8) {
+        float v[8];
+        for (int j = 0; j < 8; ++j) v[j] = x[min(i + 256 * j, K - 1)];
+        for (int j = 0; j < 8; ++j)
+            if (i + 256 * j < K) s += v[j] * v[j];
+    }
+    return s;
+}
+template <int LS = 1>
+__device__ __forceinline__ void q8_store(const float* v, int g, uint8_t* xa, int K, int m, int b, bool live = true);
 __device__ __forceinline__ void q8_zero(int g, uint8_t* xa, int K, int m, int b);
 
 // Four lanes per 32-block: lane part g holds the block's elements {4g..4g+3, 16+4g..16+4g+3}, which is exactly its
@@ -110,24 +122,24 @@ __global__ __launch_bounds__(256) void k_quant_act(const float* __restrict__ X, 
     // whatever the row holds reaches only output rows that nothing reads.
     if (src < 0) return;
     const float* x = X + (size_t) src * ldx;
-    float scale = 1.0f;
-    if (nw) {
-        float s = 0.0f;
-        for (int i = t; i < K; i += 256) s += x[i] * x[i];
-        s = block_reduce_sum256(s, red);
-        scale = 1.0f / sqrtf(s / (float) K + eps);
-    }
     const int nbp = xa_nbp(K);
     const int b = blockIdx.y * 64 + (t >> 2), g = t & 3;
+    // the block's values and norm weights are loaded beside the row's sum (block clamped: no load behind a branch)
+    const int e0 = 32 * min(b, nb - 1) + 4 * g;
+    const float4 lo4 = *(const float4*) (x + e0), hi4 = *(const float4*) (x + e0 + 16);
+    float4 wl = {1.f, 1.f, 1.f, 1.f}, wh = wl;
+    float scale = 1.0f;
+    if (nw) {
+        wl = *(const float4*) (nw + e0), wh = *(const float4*) (nw + e0 + 16);
+        scale = 1.0f / sqrtf(block_reduce_sum256(row_squares(x, K, t), red) / (float) K + eps);
+    }
     if (b >= nbp) return;  // (whole 4-lane groups leave together: the shuffles below stay within a group)
     if (b >= nb) {  // a padding block of the last 4-block group: zero
         q8_zero(g, xa, K, m, b);
         return;
     }
-    const float4 lo4 = *(const float4*) (x + 32 * b + 4 * g), hi4 = *(const float4*) (x + 32 * b + 16 + 4 * g);
     float v[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
     if (nw) {
-        const float4 wl = *(const float4*) (nw + 32 * b + 4 * g), wh = *(const float4*) (nw + 32 * b + 16 + 4 * g);
         const float w[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
         for (int j = 0; j < 8; ++j) v[j] = (v[j] * scale) * w[j];
     }
@@ -139,15 +151,77 @@ __global__ __launch_bounds__(256) void k_quant_act(const float* __restrict__ X, 
     q8_store(v, g, xa, K, m, b);
 }
 
+// The same of many rows, a 16-row tile a workgroup of 16 wavefronts (and a share of its blocks, grid y): a wavefront
+// takes a (tile, block), lane m + 16 g row m's lane part g, so it reads whole 128-byte lines and writes the block's
+// fragment as 1 KB and its scales and corrections as 64 bytes each. (A row a workgroup, the 16-byte pieces of a
+// fragment's lines come from workgroups on all 8 XCDs: 2048 rows of 2560 with a norm 22.8 us, 2304 of 2048 without
+// 14.6.) The row sums are the row kernel's.
+__global__ __launch_bounds__(1024) void k_quant_act_tile(const float* __restrict__ X, const int32_t* __restrict__ rows,
+                                                         int M, int K, int ldx, const float* __restrict__ nw, float eps,
+                                                         uint8_t* __restrict__ xa, float* __restrict__ xn, int ldn) {
+    __shared__ float red[16][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m0 = blockIdx.x * 16;
+    const int nb = K / 32, nbp = xa_nbp(K);
+    if (nw) {
+        // 256 threads (q) take rows 4 q .. 4 q + 3 together: thread t each row's elements t, t + 256, ... in order
+        const int q = threadIdx.x >> 8, t = threadIdx.x & 255;
+        const float* xr[4];
+        float sq[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int p = 0; p < 4; ++p) {
+            const int mr = min(m0 + 4 * q + p, M - 1);
+            xr[p] = X + (size_t) max(rows ? rows[mr] : mr, 0) * ldx;
+        }
+        for (int i = t; i < K; i += 256 * 4) {
+            float v[4][4];
+            for (int j = 0; j < 4; ++j)
+                for (int p = 0; p < 4; ++p) v[p][j] = xr[p][min(i + 256 * j, K - 1)];
+            for (int j = 0; j < 4; ++j)
+                if (i + 256 * j < K)
+                    for (int p = 0; p < 4; ++p) sq[p] += v[p][j] * v[p][j];
+        }
+        for (int p = 0; p < 4; ++p) {
+            for (int o = 32; o > 0; o >>= 1) sq[p] += __shfl_xor(sq[p], o);
+            if (lane == 0) red[4 * q + p][wave & 3] = sq[p];
+        }
+        __syncthreads();
+    }
+    const int r = lane & 15, g = lane >> 4, m = m0 + r;
+    const int src = m < M ? (rows ? rows[m] : m) : -1;  // (rows past M and padding rows of an expert's tile: not written)
+    const float* x = X + (size_t) max(src, 0) * ldx;
+    const float scale = nw ? 1.0f / sqrtf(((red[r][0] + red[r][1]) + (red[r][2] + red[r][3])) / (float) K + eps) : 1.0f;
+    for (int b = blockIdx.y * 16 + wave; b < nbp; b += 16 * gridDim.y) {
+        float v[8];
+        if (b < nb) {
+            const int e0 = 32 * b + 4 * g;
+            const float4 lo4 = *(const float4*) (x + e0), hi4 = *(const float4*) (x + e0 + 16);
+            const float l8[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+            for (int j = 0; j < 8; ++j) v[j] = l8[j];
+            if (nw) {
+                const float4 wl = *(const float4*) (nw + e0), wh = *(const float4*) (nw + e0 + 16);
+                const float w[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
+                for (int j = 0; j < 8; ++j) v[j] = (v[j] * scale) * w[j];
+            }
+            if (xn && src >= 0) {
+                float* o = xn + (size_t) m * ldn + 32 * b;
+                *(float4*) (o + 4 * g) = (float4){v[0], v[1], v[2], v[3]};
+                *(float4*) (o + 16 + 4 * g) = (float4){v[4], v[5], v[6], v[7]};
+            }
+        }
+        if (b < nb) q8_store<16>(v, g, xa, K, m, b, src >= 0);
+        else if (src >= 0) q8_zero(g, xa, K, m, b);
+    }
+}
+
 // Row m, block b of a Q8_0 operand from its 32 fp32 values (this lane's 8: elements 4g..4g+3, 16+4g..16+4g+3):
 // ggml x86 quantize_row_q8_0, d = amax / 127 (stored fp16), q = round-half-even(x * 127 / amax). The 4 lanes of a
-// block are adjacent (the shuffles stay within them). Writes the lane's fragment slice (q, and q / 16 for elements
+// block are LS apart (the shuffles stay within them). Writes the lane's fragment slice (q, and q / 16 for elements
 // 16..31) and, from lane part 0, the block's scale and corrections (see sn_common.h).
-__device__ __forceinline__ void q8_store(const float* v, int g, uint8_t* xa, int K, int m, int b) {
+template <int LS>
+__device__ __forceinline__ void q8_store(const float* v, int g, uint8_t* xa, int K, int m, int b, bool live) {
     float amax = 0.0f;
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    amax = fmaxf(amax, __shfl_xor(amax, 2));
+    amax = fmaxf(amax, __shfl_xor(amax, LS));
+    amax = fmaxf(amax, __shfl_xor(amax, 2 * LS));
     const float d = amax / 127.f;
     const float id = (amax != 0.0f) ? 127.f / amax : 0.0f;
     half8 q;
@@ -158,10 +232,11 @@ __device__ __forceinline__ void q8_store(const float* v, int g, uint8_t* xa, int
         if (j < 4) slo += r;
         else shi += r;
     }
-    slo += __shfl_xor(slo, 1);
-    shi += __shfl_xor(shi, 1);
-    slo += __shfl_xor(slo, 2);
-    shi += __shfl_xor(shi, 2);
+    slo += __shfl_xor(slo, LS);
+    shi += __shfl_xor(shi, LS);
+    slo += __shfl_xor(slo, 2 * LS);
+    shi += __shfl_xor(shi, 2 * LS);
+    if (!live) return;
     uint8_t* rec = xa + xa_rec_off(K, m, b);
     *(half8*) (rec + (b & 3) * 1024 + 16 * ((m & 15) + 16 * g)) = q;
     if (g == 0) {
@@ -1941,6 +2016,16 @@ int swiglu_quant(const float* part, int ks, int M, int F, float* h, uint8_t* xa,
 void quant_act(const float* x, const int32_t* rows, int M, int K, int ldx, const float* nw, float eps, uint8_t* xa,
                float* xn, int ldn, hipStream_t st) {
     if (M <= 0) return;
+    // A tile a workgroup from 10 MB of rows with a norm (each of a tile's grid.y workgroups sums its 16 rows, so no more
+    // than fill the chip once: 2560 wide, row / tile kernel: 256 rows 5.4 / 6.5 us, 512 7.1 / 6.8, 2048 21 / 10.5), from
+    // 1.3 MB without (128 rows 3.1 / 3.2, 512 5.3 / 3.6, 2048 15.1 / 7.3).
+    const long mk = (long) M * K;
+    if (mk >= (nw ? 1250000 : 320000) && M >= 16) {
+        const int mt = (M + 15) / 16, ny = (xa_nbp(K) + 15) / 16;
+        const dim3 grid(mt, nw ? std::max(1, std::min(ny, 256 / mt)) : ny);
+        hipLaunchKernelGGL(k_quant_act_tile, grid, dim3(1024), 0, st, x, rows, M, K, ldx, nw, eps, xa, xn, ldn);
+        return;
+    }
     hipLaunchKernelGGL(k_quant_act, dim3(M, (xa_nbp(K) + 63) / 64), dim3(256), 0, st, x, rows, M, K, ldx, nw, eps, xa,
                        xn, ldn);
 }

@@ -69,3 +69,23 @@ def test_many_rows_are_the_few_rows_bits(wt, M, N, K, epi, pad, off):
         want[off + m * ldy:off + m * ldy + n * ldy] = matmul(L, wt, w, x[m:m + n], N, epi, ldy, part)
     got = matmul(L, wt, w, x, N, epi, ldy, y0, off)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("M,K,norm", [(160, 2016, False), (131, 2560, False), (489, 2560, True), (613, 2080, True), (33, 9728, False)])
+def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
+    """The activation quantizer's tile form (ragged last tiles, K not a multiple of 128, with and without the norm)
+    against calls of 16 rows: the same integers and scales."""
+    L, r = S.lib(), np.random.default_rng(M + K)
+    x = (r.standard_normal((M, K)) * np.exp(r.standard_normal((M, 1)))).astype(np.float32)
+    nw = U.dev((1 + 0.1 * r.standard_normal(K)).astype(np.float32))
+
+    def operand(rows):
+        xa = U.empty(L.snk_xa_bytes(len(rows), K))
+        assert L.snk_quant_act(U.ptr(U.dev(rows)), len(rows), K, K, U.ptr(nw) if norm else None, 1e-6, U.ptr(xa),
+                               U.stream()) == 0
+        return U.xa_decode(U.host(xa, np.uint8), len(rows), K)
+
+    q, d = operand(x)
+    for m in range(0, M, 16):
+        wq, wd = operand(x[m:m + 16])
+        assert np.array_equal(q[m:m + 16], wq) and np.array_equal(d[m:m + 16].view(np.uint32), wd.view(np.uint32))
