@@ -248,7 +248,16 @@ __device__ __forceinline__ AmxPart amx_shfl(AmxPart p, int o) {
     q.pad = 0.0f;
     return q;
 }
+// the chosen id alone (no record asked for): 2 of the 7 values exchanged
+__device__ __forceinline__ AmxPart amx_best(AmxPart p, float best, int idx) {
+    if (better(best, idx, p.best, p.idx)) p.best = best, p.idx = idx;
+    return p;
+}
 __device__ __forceinline__ AmxPart amx_wave(AmxPart p, bool lse) {
+    if (!lse) {
+        for (int o = 32; o > 0; o >>= 1) p = amx_best(p, __shfl_xor(p.best, o), __shfl_xor(p.idx, o));
+        return p;
+    }
     for (int o = 32; o > 0; o >>= 1) p = amx_merge(p, amx_shfl(p, o), lse);
     return p;
 }
@@ -275,11 +284,13 @@ __global__ __launch_bounds__(256) void k_argmax_part(const float* __restrict__ l
         const int i = i0 + 256 * k;
         if (i >= V) break;
         bool b = false;
-        for (int j = 0; j < 8; ++j) b = b || i == bn[j];
+        if (nb > 0)  // (uniform)
+            for (int j = 0; j < 8; ++j) b = b || i == bn[j];
         if (!b && (p.idx == 0x7fffffff || v[k] > p.best)) {
             p.best = v[k];
             p.idx = i;
         }
+        if (!LSE) continue;
         if (v[k] > p.tp.m1) {
             p.tp.m2 = p.tp.m1;
             p.tp.i2 = p.tp.i1;
@@ -297,7 +308,7 @@ __global__ __launch_bounds__(256) void k_argmax_part(const float* __restrict__ l
     if (lane == 0) sp[w] = p;
     __syncthreads();
     if (t == 0) {
-        for (int k = 1; k < 4; ++k) p = amx_merge(p, sp[k], LSE);
+        for (int k = 1; k < 4; ++k) p = LSE ? amx_merge(p, sp[k], true) : amx_best(p, sp[k].best, sp[k].idx);
         part[(size_t) r * nch + c] = p;
     }
 }
@@ -307,7 +318,10 @@ __global__ __launch_bounds__(64) void k_argmax_fin(const AmxPart* __restrict__ p
                                                    float* __restrict__ rec) {
     const int r = blockIdx.x, lane = threadIdx.x;
     AmxPart p = {-INFINITY, 0x7fffffff, {-INFINITY, 0x7fffffff, -INFINITY, 0x7fffffff}, 0.0f, 0.0f};
-    for (int c = lane; c < nch; c += 64) p = amx_merge(p, part[(size_t) r * nch + c], LSE);
+    for (int c = lane; c < nch; c += 64) {
+        const AmxPart* q = part + (size_t) r * nch + c;
+        p = LSE ? amx_merge(p, *q, true) : amx_best(p, q->best, q->idx);
+    }
     p = amx_wave(p, LSE);
     if (lane != 0) return;
     const int idx = p.idx == 0x7fffffff ? -1 : p.idx;

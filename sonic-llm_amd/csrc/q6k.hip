@@ -112,34 +112,49 @@ __global__ __launch_bounds__(64) void k_q6k_dequant(const uint8_t* __restrict__ 
 }
 
 // ---- Q8_K activation records ----------------------------------------------------------------------------------------
-// grid (rows M), 256 threads: row m (source rows[m] of X when given) RMS-normed by nw when given (scale 1/sqrt(mean
-// x^2 + eps), summed as the activation quantizer does: thread t over elements t, t + 256, ..), then wavefront w
-// quantizes blocks w, w + 4, .. with lane l holding elements 4 l .. 4 l + 3: ggml quantize_row_q8_K_ref (max = the
+// grid (rows M), a wavefront a block of the row (4 to 16): row m (source rows[m] of X when given) RMS-normed by nw when
+// given (scale 1/sqrt(mean x^2 + eps), summed by the first 256 threads as the activation quantizer does: thread t over
+// elements t, t + 256, ..), then each wavefront quantizes its block (and those 16 on) with lane l holding elements
+// 4 l .. 4 l + 3 (32 rows of 2560: 4.1 us; 4 wavefronts a row that loaded
+// after the sum: 6.8): ggml quantize_row_q8_K_ref (max = the
 // value of largest |x|, the first on ties; iscale = -127 / max; q = min(127, round-half-even(iscale * x)); d =
 // 1 / iscale; an all-zero block: d = 0, q = 0).
-__global__ __launch_bounds__(256) void k_quant_q8k(const float* __restrict__ X, const int32_t* __restrict__ rows,
+__global__ __launch_bounds__(1024) void k_quant_q8k(const float* __restrict__ X, const int32_t* __restrict__ rows,
                                                    int K, int ldx, const float* __restrict__ nw, float eps,
                                                    uint8_t* __restrict__ xk) {
     __shared__ float red_s[4];
-    const int m = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int m = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6, nwv = blockDim.x >> 6, nb = K / 256;
     const float* x = X + (size_t) (rows ? rows[m] : m) * ldx;
+    // the wavefront's first block is loaded beside the row's sum (clamped: no load behind a branch)
+    const int f0 = 256 * min(wv, nb - 1) + 4 * lane;
+    float x0[4], w0[4] = {1.f, 1.f, 1.f, 1.f};
+    for (int i = 0; i < 4; ++i) x0[i] = x[f0 + i];
     float scale = 1.0f;
     if (nw) {
-        float s = 0.0f;
-        for (int i = t; i < K; i += 256) s += x[i] * x[i];
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-        if (lane == 0) red_s[wv] = s;
+        for (int i = 0; i < 4; ++i) w0[i] = nw[f0 + i];
+        if (wv < 4) {
+            float s = 0.0f;
+            for (int i = t; i < K; i += 256 * 8) {
+                float v[8];
+                for (int j = 0; j < 8; ++j) v[j] = x[min(i + 256 * j, K - 1)];
+                for (int j = 0; j < 8; ++j)
+                    if (i + 256 * j < K) s += v[j] * v[j];
+            }
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+            if (lane == 0) red_s[wv] = s;
+        }
         __syncthreads();
-        s = (red_s[0] + red_s[1]) + (red_s[2] + red_s[3]);
+        const float s = (red_s[0] + red_s[1]) + (red_s[2] + red_s[3]);
         scale = 1.0f / sqrtf(s / (float) K + eps);
     }
-    for (int b = wv; b < K / 256; b += 4) {
+    for (int b = wv; b < nb; b += nwv) {
         const int e0 = 256 * b + 4 * lane;
         float v[4];
         float a = 0.0f, va = 0.0f;
         int ia = 1 << 30;
         for (int i = 0; i < 4; ++i) {
-            v[i] = nw ? (x[e0 + i] * scale) * nw[e0 + i] : x[e0 + i];
+            const float xv = b == wv ? x0[i] : x[e0 + i];
+            v[i] = nw ? (xv * scale) * (b == wv ? w0[i] : nw[e0 + i]) : xv;
             if (fabsf(v[i]) > a) {
                 a = fabsf(v[i]);
                 ia = 4 * lane + i;
@@ -290,7 +305,7 @@ void q6k_dequant(const uint8_t* tiles, int N, int K, float* out, hipStream_t st)
 }
 void quant_q8k(const float* x, const int32_t* rows, int M, int K, int ldx, const float* nw, float eps, uint8_t* xk,
                hipStream_t st) {
-    if (M > 0) hipLaunchKernelGGL(k_quant_q8k, dim3(M), dim3(256), 0, st, x, rows, K, ldx, nw, eps, xk);
+    if (M > 0) hipLaunchKernelGGL(k_quant_q8k, dim3(M), dim3(64 * (K / 256 < 4 ? 4 : K / 256 > 16 ? 16 : K / 256)), 0, st, x, rows, K, ldx, nw, eps, xk);
 }
 int q6k_gemm(const uint8_t* tiles, const uint8_t* xk, int M, int N, int K, float* y, int ldy, hipStream_t st) {
     if (M <= 0) return 0;
