@@ -1368,25 +1368,40 @@ __global__ __launch_bounds__(256) void k_q4_gemv(GemmArgs a) {
             if (m < M) a.part[((size_t) slice * a.M + m) * a.N + col] = acc[m];
 }
 
-// k-slice partial sums added in slice order, then the epilogue
-__global__ void k_q4_reduce(GemmArgs a) {
-    const int outN = a.epi == EPI_SWIGLU ? a.N / 2 : a.N;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.M * outN) return;
-    const int row = i / outN, col = i % outN;
-    auto sum = [&](int c) {
-        float s = 0.0f;
-        for (int k = 0; k < a.ks; ++k) s += a.part[((size_t) k * a.M + row) * a.N + c];
+// k-slice partial sums added in slice order, then the epilogue: V columns a thread, KM slices' loads in flight (a loop
+// of one slice's load and add at a time waits on each in turn: 100 x 6144 of 5
+// slices 5.0 us, so 4.2; 32 x 9728 SwiGLU of 3 4.3, so 4.0).
+template <int V, int KM>
+__global__ __launch_bounds__(256) void k_q4_reduce(GemmArgs a) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const int outN = (a.epi == EPI_SWIGLU ? a.N / 2 : a.N) / V;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t row = i / (uint32_t) outN, col = V * (i % (uint32_t) outN);
+    if (row >= (uint32_t) a.M) return;
+    const size_t stride = (size_t) a.M * a.N;
+    auto sum = [&](uint32_t c) {
+        const float* p = a.part + (size_t) row * a.N + c;
+        vec s = (vec) 0.0f;
+        for (int k0 = 0; k0 < a.ks; k0 += KM) {
+            vec v[KM];
+            for (int k = 0; k < KM; ++k) v[k] = *(const vec*) (p + (size_t) min(k0 + k, a.ks - 1) * stride);
+            for (int k = 0; k < KM; ++k)
+                if (k0 + k < a.ks) s += v[k];
+        }
         return s;
     };
+    vec* y = (vec*) (a.y + (size_t) row * a.ldy + col);
     if (a.epi == EPI_SWIGLU) {
         // output column 16 p + n: gate column 32 p + n, up column 32 p + 16 + n of the interleaved matrix
-        const int p = col / 16, n = col % 16;
-        a.y[(size_t) row * a.ldy + col] = silu(sum(32 * p + n)) * sum(32 * p + 16 + n);
+        const uint32_t c = 32 * (col / 16) + col % 16;
+        const vec g = sum(c), u = sum(c + 16);
+        vec h;
+        for (int j = 0; j < V; ++j) h[j] = silu(g[j]) * u[j];
+        *y = h;
     } else if (a.epi == EPI_ADD) {
-        a.y[(size_t) row * a.ldy + col] += sum(col);
+        *y += sum(col);
     } else {
-        a.y[(size_t) row * a.ldy + col] = sum(col);
+        *y = sum(col);
     }
 }
 
@@ -1830,11 +1845,29 @@ int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, flo
     return 1;
 }
 
+// 4 columns a thread where the slices' and the output's rows are 16-byte aligned. Up to 256 workgroups' worth of
+// threads go as single wavefronts, so that a few rows still reach every CU.
+static void launch_reduce(const GemmArgs& a, hipStream_t st) {
+    const int cols = a.epi == EPI_SWIGLU ? a.N / 2 : a.N;
+    const bool v4 = a.N % 4 == 0 && a.ldy % 4 == 0 && ((uintptr_t) a.part | (uintptr_t) a.y) % 16 == 0;
+    const long n = (long) a.M * (v4 ? cols / 4 : cols);
+    const int wg = n <= 65536 ? 64 : 256;
+    const dim3 grid((unsigned) ((n + wg - 1) / wg)), block(wg);
+    if (v4) {
+        if (a.ks == 1) hipLaunchKernelGGL((k_q4_reduce<4, 1>), grid, block, 0, st, a);
+        else if (a.ks <= 4) hipLaunchKernelGGL((k_q4_reduce<4, 4>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_q4_reduce<4, 8>), grid, block, 0, st, a);
+    } else {
+        if (a.ks <= 4) hipLaunchKernelGGL((k_q4_reduce<1, 4>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_q4_reduce<1, 8>), grid, block, 0, st, a);
+    }
+}
+
 void q4_reduce_slices(const float* part, int ks, int M, int N, float* y, hipStream_t st) {
     GemmArgs a{};
     a.part = const_cast<float*>(part); a.y = y;
     a.M = M; a.N = N; a.ldy = N; a.epi = EPI_STORE; a.ks = ks;
-    hipLaunchKernelGGL(k_q4_reduce, dim3((M * N + 255) / 256), dim3(256), 0, st, a);
+    launch_reduce(a, st);
 }
 
 int q4_gemm(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* y, int ldy, int epi, float* ws,
@@ -1856,8 +1889,7 @@ int q4_gemm(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* y, 
     GemmArgs a{};
     a.part = ws; a.y = y;
     a.M = M; a.N = N; a.K = K; a.ldy = ldy; a.epi = epi; a.ks = ks;
-    const int tot = M * (epi == EPI_SWIGLU ? N / 2 : N);
-    hipLaunchKernelGGL(k_q4_reduce, dim3((tot + 255) / 256), dim3(256), 0, st, a);
+    launch_reduce(a, st);
     return 0;
 }
 

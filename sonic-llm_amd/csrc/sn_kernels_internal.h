@@ -71,7 +71,7 @@ static inline int fe_slice_index(int ks) {
 // slices are the same for both, so a row's sums do not depend on the kernel.
 struct GemmPlan {
     int nstripes, ngroups, spw, sets, ks, gps;
-    bool stream;    // the streaming kernel serves this matrix below Q4_PAIR_ROWS rows
+    bool stream;    // the streaming kernel serves this matrix below the many-row kernel's rows
     int sspw, smt;  // its stripes a wavefront and row tiles a workgroup
     int sd;         // its ring depth (groups of weights in flight a wavefront)
 };

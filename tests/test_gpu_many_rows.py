@@ -89,3 +89,53 @@ def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
     for m in range(0, M, 16):
         wq, wd = operand(x[m:m + 16])
         assert np.array_equal(q[m:m + 16], wq) and np.array_equal(d[m:m + 16].view(np.uint32), wd.view(np.uint32))
+
+
+@pytest.mark.parametrize("M,N,K,epi,pad,off", [
+    (1, 64, 32, STORE, 0, 0),          # one slice
+    (3, 4, 4096, ADD, 0, 0),           # one thread a row
+    (5, 1001, 4096, STORE, 0, 0),      # columns not a multiple of 4: the scalar form
+    (7, 1000, 4096, ADD, 3, 0),        # rows of y unaligned: the scalar form
+    (7, 1000, 4096, ADD, 4, 0),
+    (17, 2560, 9728, STORE, 0, 1),     # y off 16 bytes: the scalar form
+    (17, 2560, 9728, ADD, 0, 4),
+    (2, 96, 9728, SWIGLU, 0, 0),       # most slices; F = 48
+    (2, 96, 9728, SWIGLU, 1, 0),
+    (95, 4128, 1056, SWIGLU, 0, 0),    # more than single wavefronts' worth
+])
+def test_slice_sum_epilogues(M, N, K, epi, pad, off):
+    """The slices' sum in its 4-column and scalar forms against 64-bit sums of the same integers and scales. Both sides
+    add the same K / 32 products; in 32 bits each of those and the slices' adds rounds once (the scale's product too):
+    within (K / 32 + 18) 2^-24 of the sum of their magnitudes; SwiGLU: gate and up so, |silu'| <= 1.1, its own few
+    roundings and the exponent's (|g| of them) beside."""
+    from oracle import oracle as O
+
+    L, r = S.lib(), np.random.default_rng(M * 11 + N)
+    raw = weights(r, N, K, 2)
+    w = U.empty(L.snk_q4_stripes_bytes(N, K))
+    assert L.snk_q4_repack(U.ptr(U.dev(raw)), N, K, U.ptr(w), U.stream()) == 0
+    x = r.standard_normal((M, K)).astype(np.float32)
+    ldy = (N // 2 if epi == SWIGLU else N) + pad
+    y0 = r.standard_normal(M * ldy + off + 8).astype(np.float32)
+    got = matmul(L, 2, w, x, N, epi, ldy, y0, off)
+    xa = U.empty(L.snk_xa_bytes(M, K))
+    assert L.snk_quant_act(U.ptr(U.dev(x)), M, K, K, None, 1e-6, U.ptr(xa), U.stream()) == 0
+    a = U.xa_values(U.host(xa, np.uint8), M, K).astype(np.float64)
+    b = O.dequantize_q4_0(raw.reshape(N, -1), K).reshape(N, K).astype(np.float64)
+    want, mag = a @ b.T, np.einsum("mbk,nbk->mnb", a.reshape(M, -1, 32), b.reshape(N, -1, 32))
+    mag = np.abs(mag).sum(-1) * (K // 32 + 18) * 2.0 ** -24
+    if epi == SWIGLU:  # stripes of 16 columns, gate and up in turn
+        s, m = want.reshape(M, -1, 2, 16), mag.reshape(M, -1, 2, 16)
+        g, u, dg, du = s[:, :, 0], s[:, :, 1], m[:, :, 0], m[:, :, 1]
+        sg = g / (1 + np.exp(-g))
+        want = (sg * u).reshape(M, -1)
+        mag = (1.1 * dg * (np.abs(u) + du) + np.abs(sg) * du + (8 + 2 * np.abs(g)) * 2.0 ** -24 * np.abs(sg * u) + 1e-12).reshape(M, -1)
+    y = y0.copy()
+    rows = y[off:off + M * ldy].reshape(M, ldy)
+    cols = want.shape[1]
+    base = rows[:, :cols].astype(np.float64) if epi == ADD else 0.0
+    out = got[off:off + M * ldy].reshape(M, ldy)
+    assert np.all(np.abs(out[:, :cols] - (want + base)) <= mag + 2.0 ** -23 * np.abs(want + base) + 1e-12)
+    keep = np.ones(y.size, bool)
+    keep[off:off + M * ldy].reshape(M, ldy)[:, :cols] = False
+    assert np.array_equal(got[keep], y[keep])  # nothing past the columns is written
