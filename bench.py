@@ -465,7 +465,7 @@ def bench_prefill(args):
     layer = (H + 2 * KVH) * 128 * E + E * H * 128 + 2 * F * E + E * F
     flop = 2.0 * rows * layer * cfg["n_layer"] + 2.0 * E * cfg["n_vocab"]
     g = kernels.get("gemm")
-    roof_mfma = {"kernel": "k_q4_gemm / k_q4_gemm_fk2 (the full-K walk)", "bound": "mfma", "achieved": round(flop / (g["ms_per_step"] * 1e-3) / 1e12, 1),
+    roof_mfma = {"kernel": "k_q4_gemm_w (32x32 tiles)", "bound": "mfma", "achieved": round(flop / (g["ms_per_step"] * 1e-3) / 1e12, 1),
                  "peak": MFMA_F16_PEAK / 1e12, "unit": "TFLOP/s",
                  "frac": round(flop / (g["ms_per_step"] * 1e-3) / MFMA_F16_PEAK, 4),
                  "traffic": profile_traffic("prefill_qwen3_4b_2048_rows512_traffic.json", "k_q4_gemm"),
