@@ -1416,6 +1416,8 @@ __global__ __launch_bounds__(256) void k_q4_reduce(GemmArgs a) {
 // the consumer one more partial sum to read.
 #define Q4_WIDE (8 * 768)  // stripes of an LM-head-wide matrix
 #define Q4_MANY_ROWS 256   // rows from which every matrix takes the many-row kernel
+// 32 x 32 tiles (of rows, padding not counted) from which fewer rows' gate|up takes it with its SwiGLU (q4_gemm_swiglu_fits)
+#define SWIGLU_WIDE_TILES 1200
 GemmPlan q4_plan(int N, int K, int wt) {
     GemmPlan p;
     p.nstripes = (N + 15) / 16;
@@ -1618,6 +1620,9 @@ static bool fused_shape(int M, int N, int K, int wt, int fe, int nxcd, int cnt_l
     if (M <= 0 || M >= Q4_MANY_ROWS || nxcd < 1 || (wt != WT_Q4_0 && wt != WT_Q8_0)) return false;
     p = q4_plan(N, K, wt);
     if (!p.stream || p.gps > 8) return false;
+    // (the many-row kernel and the rope kernel; a 6-layer step of the 4B shape, fused / so, us: 192 rows 965 / 960, 224
+    // 1096 / 1074, 255 1190 / 1158)
+    if (fe == FE_ROPE && wide_takes(M, p)) return false;
     // a set must hold whole epilogue units: one head (8 stripes: two a wavefront, Q4_0 tiles), or S Q8_0 blocks of
     // SwiGLU columns (64 S interleaved columns)
     if (fe == FE_ROPE) {
@@ -1824,9 +1829,13 @@ int q4_gemm_grouped_swiglu(const uint8_t* w, size_t wstride, const int32_t* item
     return 1;
 }
 
+// Below Q4_MANY_ROWS against the streaming kernel's own SwiGLU epilogue, which unpacks every weight again for each 32
+// rows and writes its slices. A 6-layer step of the 4B shape (19456 x 2560, T tiles), streaming / this, us: 48 rows
+// (T = 912) 570 / 574, 64 (1216) 619 / 611, 96 (1824) 754 / 698, 128 868 / 791, 192 1131 / 1008, 255 1393 / 1229. Fewer tiles leave SIMDs without one.
 bool q4_gemm_swiglu_fits(int M, int N, int K, int wt) {
-    if (wt != WT_Q4_0 || M < Q4_MANY_ROWS || N % 256 != 0) return false;
+    if (wt != WT_Q4_0 || N % 256 != 0) return false;
     const GemmPlan p = q4_plan(N, K, wt);
+    if (M < Q4_MANY_ROWS && (long) M * ((p.nstripes + 1) / 2) < 32 * SWIGLU_WIDE_TILES) return false;
     return p.ks > 1 && p.spw == 1 && p.gps % 2 == 0 && p.nstripes >= 384;
 }
 

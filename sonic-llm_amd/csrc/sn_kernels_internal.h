@@ -81,8 +81,8 @@ GemmPlan q4_plan(int N, int K, int wt = WT_Q4_0);
 // the raw matmul with an explicit plan (tuning): mt row tiles a workgroup, spw stripes a wavefront, G groups a slice
 // loaded at once (G 0: the default plan); the slice count, or -1
 // part[ks][M][N] added in slice order into y [M][N]
-// The prompt rows' gate|up matmul with its SwiGLU: from 256 rows, a Q4_0 stripe-interleaved matrix of N = 2F (F a
-// multiple of 128) through the many-row kernel (k_q4_gemm_w) with silu(gate) * up written as fp32 rows h [M][F] and
+// The gate|up matmul of many rows with its SwiGLU: from 256 rows, or fewer where their tiles fill the chip, a Q4_0
+// stripe-interleaved matrix of N = 2F (F a multiple of 128) through the many-row kernel (k_q4_gemm_w) with silu(gate) * up written as fp32 rows h [M][F] and
 // as the Q8_0 operand xo (K = F), the same bits as the matmul's slices through k_swiglu_quant. xo must not be xa.
 // Returns 1, or 0 when the shape does not qualify (nothing launched: use the matmul and swiglu_quant).
 int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* h, uint8_t* xo, hipStream_t st,

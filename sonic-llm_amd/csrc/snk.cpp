@@ -153,7 +153,7 @@ extern "C" int snk_q4_gemm(const void* d_stripes, const void* d_xa, int M, int N
 extern "C" int snk_q4_gemm_swiglu(const void* d_stripes, const void* d_xa, int M, int N, int K, float* d_h,
                                   void* d_xo, void* stream) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 32 || !d_h || !d_xo || d_xo == d_xa) return -1;
-    if (!q4_gemm_swiglu_fits(M, N, K, WT_Q4_0)) return 1;
+    if (M < 256 || !q4_gemm_swiglu_fits(M, N, K, WT_Q4_0)) return 1;  // (prompt rows, as the header says)
     const int rc = q4_gemm_swiglu((const uint8_t*) d_stripes, (const uint8_t*) d_xa, M, N, K, d_h, (uint8_t*) d_xo,
                                   (hipStream_t) stream, WT_Q4_0);
     return rc == 1 && hipGetLastError() == hipSuccess ? 0 : -1;

@@ -139,3 +139,27 @@ def test_slice_sum_epilogues(M, N, K, epi, pad, off):
     keep = np.ones(y.size, bool)
     keep[off:off + M * ldy].reshape(M, ldy)[:, :cols] = False
     assert np.array_equal(got[keep], y[keep])  # nothing past the columns is written
+
+
+@pytest.mark.parametrize("rows", [191, 200, 255, 257])
+def test_step_rows_around_the_many_row_launches(tmp_path, rows):
+    """A prompt step whose gate|up (and q|k|v) take the many-row kernel below 256 rows against the same rows in steps of
+    40, whose matmuls keep their fused epilogues: every sampled row's logits bit for bit."""
+    path = str(tmp_path / "m.gguf")
+    S.write_model(path, S.model_cfg(2, 2048, 16, 4, 3584, 1000), 5)
+    tok = np.random.default_rng(rows).integers(0, 1000, rows).astype(np.int32)
+
+    sampled = np.array([0, 31, 70, rows // 2, rows - 1])
+
+    def logits(step):
+        out = []
+        with S.Engine(path, slots=1, ctx=320, max_rows=272) as eng:
+            for p in range(0, rows, step):
+                n = min(step, rows - p)
+                at = sampled[(sampled >= p) & (sampled < p + n)] - p
+                eng.step(tok[p:p + n], np.zeros(n, np.int32), np.arange(p, p + n, dtype=np.int32), at, n_write=0)
+                if len(at):
+                    out.append(eng.logits(np.arange(len(at))))
+        return np.concatenate(out)
+
+    assert np.array_equal(logits(rows).view(np.uint32), logits(40).view(np.uint32))
