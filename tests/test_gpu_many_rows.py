@@ -71,6 +71,33 @@ def test_many_rows_are_the_few_rows_bits(wt, M, N, K, epi, pad, off):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("wt,N,K,M,many", [
+    (2, 256, 4096, 255, False), (8, 256, 4096, 200, False),   # narrow and deep: few tiles, a long walk
+    (2, 1024, 3072, 255, False), (2, 1024, 1536, 224, False), (8, 768, 3072, 240, False),
+    (2, 1024, 2048, 207, False), (2, 1024, 2048, 208, True),  # the line
+    (2, 768, 1024, 191, False), (2, 768, 1024, 192, True), (2, 256, 4096, 256, True),
+    (2, 2560, 4096, 192, True), (8, 6144, 2560, 200, True),
+])
+def test_below_256_rows_narrow_matrices_keep_their_split_launches(wt, N, K, M, many):
+    """Which launches a matmul takes, seen in its workspace (the split launches leave their slice sums there, the
+    many-row kernel nothing): narrow and deep matrices of 192 to 255 rows, whose few wide tiles would leave most of the
+    chip idle through the whole walk, stay split. The rows are the few rows' bits either way."""
+    L, r = S.lib(), np.random.default_rng(N + K + M)
+    w = U.empty((L.snk_q4_stripes_bytes if wt == 2 else L.snk_q8_tiles_bytes)(N, K))
+    assert (L.snk_q4_repack if wt == 2 else L.snk_q8_repack)(U.ptr(U.dev(weights(r, N, K, wt))), N, K, U.ptr(w), U.stream()) == 0
+    x = r.standard_normal((M, K)).astype(np.float32)
+    xa, y = U.empty(L.snk_xa_bytes(M, K)), U.empty(4 * M * N)
+    assert L.snk_quant_act(U.ptr(U.dev(x)), M, K, K, None, 1e-6, U.ptr(xa), U.stream()) == 0
+    nb = (L.snk_q4_workspace_bytes if wt == 2 else L.snk_q8_workspace_bytes)(M, N, K)
+    ws = torch.full((nb,), 0xA5, dtype=torch.uint8, device="cuda")
+    f = L.snk_q4_gemm if wt == 2 else L.snk_q8_gemm
+    assert f(U.ptr(w), U.ptr(xa), M, N, K, U.ptr(y), N, STORE, U.ptr(ws), nb, U.stream()) == 0
+    assert bool((ws == 0xA5).all()) == many
+    got = U.host(y, np.float32, (M, N))
+    want = matmul(L, wt, w, x[:16], N, STORE, N, np.zeros(16 * N + 8, np.float32))[:16 * N].reshape(16, N)
+    assert np.array_equal(got[:16].view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("M,K,norm", [(160, 2016, False), (131, 2560, False), (489, 2560, True), (613, 2080, True), (33, 9728, False)])
 def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
     """The activation quantizer's tile form (ragged last tiles, K not a multiple of 128, with and without the norm)
