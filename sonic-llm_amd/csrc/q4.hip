@@ -1634,9 +1634,11 @@ static bool fused_shape(int M, int N, int K, int wt, int fe, int nxcd, int cnt_l
     if (M <= 0 || M >= Q4_MANY_ROWS || nxcd < 1 || (wt != WT_Q4_0 && wt != WT_Q8_0)) return false;
     p = q4_plan(N, K, wt);
     if (!p.stream || p.gps > 8) return false;
-    // (the many-row kernel and the rope kernel; a 6-layer step of the 4B shape, fused / so, us: 192 rows 965 / 960, 224
-    // 1096 / 1074, 255 1190 / 1158)
-    if (fe == FE_ROPE && wide_takes(M, p)) return false;
+    // Q|k|v of more rows: the many-row kernel and the rope kernel, whose extra launch (5 to 9 us) the faster matmul has
+    // to earn back: from 1e9 products. A 6-layer step, us, fused / so: 4096 x 1024 at 192 rows (0.8e9) 459 / 475, 224
+    // 491 / 497, 240 (1.0e9) 501 / 499, 255 509 / 505; 5120 x 2048 at 192 (2.0e9) 788 / 757, 255 893 / 865; 6144 x 2560
+    // at 192 (3.0e9) 979 / 960, 224 1124 / 1096, 255 1209 / 1166.
+    if (fe == FE_ROPE && wide_takes(M, p) && (long) M * N * K >= 1000000000L) return false;
     // a set must hold whole epilogue units: one head (8 stripes: two a wavefront, Q4_0 tiles), or S Q8_0 blocks of
     // SwiGLU columns (64 S interleaved columns)
     if (fe == FE_ROPE) {

@@ -190,3 +190,24 @@ def test_step_rows_around_the_many_row_launches(tmp_path, rows):
         return np.concatenate(out)
 
     assert np.array_equal(logits(rows).view(np.uint32), logits(40).view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,split", [(192, False), (238, False), (239, True), (255, True)])
+def test_rope_epilogue_of_a_narrow_model(tmp_path, rows, split):
+    """Q|k|v of a model of width 1024 (4096 x 1024) keeps its RoPE epilogue until the many-row matmul earns the rope
+    launch back (1e9 products: 239 rows); the sampled rows' logits are those of steps of 40 either way."""
+    path = str(tmp_path / "m.gguf")
+    S.write_model(path, S.model_cfg(2, 1024, 16, 8, 3072, 1000), 5)
+    tok = np.random.default_rng(rows).integers(0, 1000, rows).astype(np.int32)
+    out = []
+    for step in (rows, 40):
+        with S.Engine(path, slots=1, ctx=320, max_rows=256) as eng:
+            for p in range(0, rows, step):
+                n = min(step, rows - p)
+                eng.prof(step == rows)
+                eng.step(tok[p:p + n], np.zeros(n, np.int32), np.arange(p, p + n, dtype=np.int32),
+                         np.array([n - 1], np.int32), n_write=0)
+            if step == rows:
+                assert (eng.prof_read()["rope"]["launches"] > 0) == split
+            out.append(eng.logits([0]).copy())
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
