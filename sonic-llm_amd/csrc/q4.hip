@@ -162,6 +162,7 @@ __global__ __launch_bounds__(1024) void k_quant_act_tile(const float* __restrict
     __shared__ float red[16][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m0 = blockIdx.x * 16;
     const int nb = K / 32, nbp = xa_nbp(K);
+    if (m0 >= M) return;  // (the grid's padding)
     if (nw) {
         // 256 threads (q) take rows 4 q .. 4 q + 3 together: thread t each row's elements t, t + 256, ... in order
         const int q = threadIdx.x >> 8, t = threadIdx.x & 255;
@@ -2073,13 +2074,15 @@ int swiglu_quant(const float* part, int ks, int M, int F, float* h, uint8_t* xa,
 void quant_act(const float* x, const int32_t* rows, int M, int K, int ldx, const float* nw, float eps, uint8_t* xa,
                float* xn, int ldn, hipStream_t st) {
     if (M <= 0) return;
-    // A tile a workgroup from 10 MB of rows with a norm (each of a tile's grid.y workgroups sums its 16 rows, so no more
-    // than fill the chip once: 2560 wide, row / tile kernel: 256 rows 5.4 / 6.5 us, 512 7.1 / 6.8, 2048 21 / 10.5), from
-    // 1.3 MB without (128 rows 3.1 / 3.2, 512 5.3 / 3.6, 2048 15.1 / 7.3).
+    // A tile a workgroup from 5 MB of rows with a norm (2560 wide, row / tile kernel: 256 rows 5.4 / 6.5 us, 512 7.1 /
+    // 6.8, 2048 21 / 10.5), from 1.3 MB without (128 rows 3.1 / 3.2, 512 5.3 / 3.6, 2048 15.1 / 7.3).
+    // With a norm each of a tile's grid.y workgroups sums its 16 rows: no more of them than fill the chip once, and all
+    // on the tile's XCD, whose L2 then serves the rows again (the tiles padded to a multiple of 8: with 31 or 33 tiles,
+    // a tile's workgroups on all XCDs, 496 rows of 4096 took 14.5 us, 520 14.8; so 7.9 and 8.9).
     const long mk = (long) M * K;
     if (mk >= (nw ? 1250000 : 320000) && M >= 16) {
-        const int mt = (M + 15) / 16, ny = (xa_nbp(K) + 15) / 16;
-        const dim3 grid(mt, nw ? std::max(1, std::min(ny, 256 / mt)) : ny);
+        const int mt = (M + 15) / 16, mt8 = (mt + 7) / 8 * 8, ny = (xa_nbp(K) + 15) / 16;
+        const dim3 grid(nw ? mt8 : mt, nw ? std::max(1, std::min(ny, 256 / mt8)) : ny);
         hipLaunchKernelGGL(k_quant_act_tile, grid, dim3(1024), 0, st, x, rows, M, K, ldx, nw, eps, xa, xn, ldn);
         return;
     }

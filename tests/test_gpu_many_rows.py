@@ -98,7 +98,8 @@ def test_below_256_rows_narrow_matrices_keep_their_split_launches(wt, N, K, M, m
     assert np.array_equal(got[:16].view(np.uint32), want.view(np.uint32))
 
 
-@pytest.mark.parametrize("M,K,norm", [(160, 2016, False), (131, 2560, False), (489, 2560, True), (613, 2080, True), (33, 9728, False)])
+@pytest.mark.parametrize("M,K,norm", [(160, 2016, False), (131, 2560, False), (489, 2560, True), (613, 2080, True), (33, 9728, False),
+                                      (520, 4096, True), (331, 5120, True)])
 def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
     """The activation quantizer's tile form (ragged last tiles, K not a multiple of 128, with and without the norm)
     against calls of 16 rows: the same integers and scales."""
@@ -116,6 +117,39 @@ def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
     for m in range(0, M, 16):
         wq, wd = operand(x[m:m + 16])
         assert np.array_equal(q[m:m + 16], wq) and np.array_equal(d[m:m + 16].view(np.uint32), wd.view(np.uint32))
+
+
+def test_operand_of_ragged_rows_costs_what_whole_tiles_do():
+    """A row tile's workgroups share its rows in one L2 whatever the number of tiles: 520 rows of 4096 with the norm (33
+    tiles) take about the time of 512 (32), not that of every XCD reading every row (1.8 times). Times of 20 calls as one
+    graph, the least of 12 replays in turn."""
+    L, K = S.lib(), 4096
+    nw = torch.ones(K, device="cuda")
+    graphs, keep = [], []
+    for M in (512, 520):
+        x, xa = torch.randn(M, K, device="cuda"), U.empty(L.snk_xa_bytes(M, K))
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            call = lambda: L.snk_quant_act(U.ptr(x), M, K, K, U.ptr(nw), 1e-6, U.ptr(xa), U.stream())
+            assert call() == 0
+            s.synchronize()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                for _ in range(20):
+                    assert call() == 0
+        graphs.append(g)
+        keep.append((x, xa))
+    best = [float("inf")] * 2
+    for _ in range(12):
+        for i, g in enumerate(graphs):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            g.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], a.elapsed_time(b))
+    print("512 rows %.2f us, 520 rows %.2f us" % tuple(50 * t for t in best))
+    assert best[1] < 1.45 * best[0]
 
 
 @pytest.mark.parametrize("M,N,K,epi,pad,off", [
