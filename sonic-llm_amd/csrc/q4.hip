@@ -2074,13 +2074,16 @@ int swiglu_quant(const float* part, int ks, int M, int F, float* h, uint8_t* xa,
 void quant_act(const float* x, const int32_t* rows, int M, int K, int ldx, const float* nw, float eps, uint8_t* xa,
                float* xn, int ldn, hipStream_t st) {
     if (M <= 0) return;
-    // A tile a workgroup from 5 MB of rows with a norm (2560 wide, row / tile kernel: 256 rows 5.4 / 6.5 us, 512 7.1 /
-    // 6.8, 2048 21 / 10.5), from 1.3 MB without (128 rows 3.1 / 3.2, 512 5.3 / 3.6, 2048 15.1 / 7.3).
+    // A tile a workgroup (row / tile kernel, us): with a norm from 1.6e6 values (6.4 MB) of 320 rows or more: 2560 wide,
+    // 520 rows 6.8 / 7.0, 640 7.5 / 7.1, 2048 21 / 10.5; 2048 wide, 700 rows 6.4 / 6.6, 900 7.5 / 6.9; 4096 wide, 384
+    // 7.2 / 7.7, 417 8.2 / 7.9; 6144 wide, 256 7.4 / 8.7, 333 9.7 / 10.0; 9728 wide, 256 11.4 / 12.5, 333 17.9 / 12.7.
+    // Without one from 400,000: 2560 wide, 140 rows 3.3 / 3.4, 175 3.6 / 3.5, 2048 15.6 / 7.5; 512 wide, 703 3.3 / 3.4,
+    // 878 3.6 / 3.4; 9728 wide, 37 3.4 / 3.5, 53 3.8 / 3.5.
     // With a norm each of a tile's grid.y workgroups sums its 16 rows: no more of them than fill the chip once, and all
     // on the tile's XCD, whose L2 then serves the rows again (the tiles padded to a multiple of 8: with 31 or 33 tiles,
     // a tile's workgroups on all XCDs, 496 rows of 4096 took 14.5 us, 520 14.8; so 7.9 and 8.9).
     const long mk = (long) M * K;
-    if (mk >= (nw ? 1250000 : 320000) && M >= 16) {
+    if (M >= (nw ? 320 : 16) && mk >= (nw ? 1600000 : 400000)) {
         const int mt = (M + 15) / 16, mt8 = (mt + 7) / 8 * 8, ny = (xa_nbp(K) + 15) / 16;
         const dim3 grid(nw ? mt8 : mt, nw ? std::max(1, std::min(ny, 256 / mt8)) : ny);
         hipLaunchKernelGGL(k_quant_act_tile, grid, dim3(1024), 0, st, x, rows, M, K, ldx, nw, eps, xa, xn, ldn);

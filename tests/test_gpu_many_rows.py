@@ -99,7 +99,8 @@ def test_below_256_rows_narrow_matrices_keep_their_split_launches(wt, N, K, M, m
 
 
 @pytest.mark.parametrize("M,K,norm", [(160, 2016, False), (131, 2560, False), (489, 2560, True), (613, 2080, True), (33, 9728, False),
-                                      (520, 4096, True), (331, 5120, True)])
+                                      (160, 2560, False), (199, 2016, False), (43, 9728, False), (625, 2560, True),
+                                      (771, 2080, True), (520, 4096, True), (331, 5120, True)])
 def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
     """The activation quantizer's tile form (ragged last tiles, K not a multiple of 128, with and without the norm)
     against calls of 16 rows: the same integers and scales."""
