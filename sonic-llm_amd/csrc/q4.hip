@@ -1848,11 +1848,14 @@ int q4_gemm_grouped_swiglu(const uint8_t* w, size_t wstride, const int32_t* item
 
 // Below Q4_MANY_ROWS against the streaming kernel's own SwiGLU epilogue, which unpacks every weight again for each 32
 // rows and writes its slices. A 6-layer step of the 4B shape (19456 x 2560, T tiles), streaming / this, us: 48 rows
-// (T = 912) 570 / 574, 64 (1216) 619 / 611, 96 (1824) 754 / 698, 128 868 / 791, 192 1131 / 1008, 255 1393 / 1229. Fewer tiles leave SIMDs without one.
+// (T = 912) 570 / 574, 64 (1216) 619 / 611, 96 (1824) 754 / 698, 128 868 / 791, 192 1131 / 1008, 255 1393 / 1229. Fewer
+// tiles leave SIMDs without one. Up to 32 rows both unpack once, and the streaming kernel stays however wide the matrix
+// (2 layers of 51200 x 5120 at 24 rows 366 / 386, at 32 378 / 394).
+// (ks > 1, an even gps and 384 stripes: the plans that had this epilogue before; others were not measured with it)
 bool q4_gemm_swiglu_fits(int M, int N, int K, int wt) {
     if (wt != WT_Q4_0 || N % 256 != 0) return false;
     const GemmPlan p = q4_plan(N, K, wt);
-    if (M < Q4_MANY_ROWS && (long) M * ((p.nstripes + 1) / 2) < 32 * SWIGLU_WIDE_TILES) return false;
+    if (M < Q4_MANY_ROWS && (M <= 32 || (long) M * ((p.nstripes + 1) / 2) < 32 * SWIGLU_WIDE_TILES)) return false;
     return p.ks > 1 && p.spw == 1 && p.gps % 2 == 0 && p.nstripes >= 384;
 }
 

@@ -246,3 +246,30 @@ def test_rope_epilogue_of_a_narrow_model(tmp_path, rows, split):
                 assert (eng.prof_read()["rope"]["launches"] > 0) == split
             out.append(eng.logits([0]).copy())
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+def test_gate_up_of_a_wide_model_up_to_32_rows(tmp_path):
+    """The widest gate|up (51200 columns: enough tiles for the many-row kernel at 24 rows) stays on the streaming kernel
+    up to 32 rows, seen without the fused epilogues as one SwiGLU launch more than at 33; the same bits as steps of 11."""
+    path = str(tmp_path / "m.gguf")
+    S.write_model(path, S.model_cfg(1, 2048, 16, 4, 25600, 1000), 5)
+    tok = np.random.default_rng(1).integers(0, 1000, 33).astype(np.int32)
+    launches = {}
+    with S.Engine(path, slots=40, ctx=64, max_rows=64) as eng:
+        eng.graphs(False)
+        eng.fuse(False)
+        want = None
+        for step in (11, 24, 32, 33):
+            eng.clear(0, 0, 33)
+            out = []
+            for p in range(0, 33, step):
+                n = min(step, 33 - p)
+                eng.prof(True)
+                eng.step(tok[p:p + n], np.zeros(n, np.int32), np.arange(p, p + n, dtype=np.int32), np.arange(n), n_write=0)
+                launches.setdefault(n, eng.prof_read()["quant"]["launches"])
+                eng.prof(False)
+                out.append(eng.logits(np.arange(n)).copy())
+            got = np.concatenate(out).view(np.uint32)
+            want = got if want is None else want
+            assert np.array_equal(got, want), step
+    assert launches[24] == launches[32] == launches[33] + 1, launches
