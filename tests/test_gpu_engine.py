@@ -432,14 +432,14 @@ def test_attention_list_forms_give_the_same_steps(tiny):
 
 def test_prompt_chunking_does_not_change_the_next_row(tmp_path):
     """A prompt fed in one step or in several gives the same cells and so the same next row, bit for bit (qbench.m's
-    read_chunks, qbench.m:124-130): 600 prompt rows in one step (the full-K matmul walk and run items at 600 rows),
-    in 200-row steps (the split launches and chunk items; the workgroup-per-row QK-RoPE adding the k-slice sums), and
-    in 64 + 536 (the 64 rows through the wavefront-per-head QK-RoPE), then the same decode row. The model's
+    read_chunks, qbench.m:124-130): 600 prompt rows in one step (the many-row matmul and run items at 600 rows),
+    in 200-row steps (q|k|v with its RoPE epilogue, the down projection split, chunk items), and in 64 + 536 (a step of
+    decode-sized launches before one of many rows), then the same decode row. The model's
     matrices all split K (n_embd 1024: 2 slices) and its gate|up is wide enough (n_ff 3072: 384 stripes) for the prompt
     SwiGLU epilogue."""
     path = str(tmp_path / "w.gguf")
     S.write_model(path, S.model_cfg(n_layer=2, n_embd=1024, n_head=8, n_head_kv=2, n_ff=3072, n_vocab=1000), seed=13)
-    assert S.q4_plan(2 * 3072, 1024)[1] > 1 and S.q4_plan(1024, 3072)[1] > 1  # (k-slices: the full-K walk applies)
+    assert S.q4_plan(2 * 3072, 1024)[1] > 1 and S.q4_plan(1024, 3072)[1] > 1  # (k-slices to add)
     r = np.random.default_rng(14)
     toks = r.integers(0, 1000, 600).astype(np.int32)
     nxt = np.array([int(r.integers(0, 1000))], np.int32)

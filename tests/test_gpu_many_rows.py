@@ -44,6 +44,8 @@ CASES = [  # wt, M, N, K, epi, ldy - columns, offset of y in floats
     (2, 192, 6144, 2560, STORE, 0, 0),      # below 256 rows
     (2, 100, 19456, 1056, SWIGLU, 0, 0),    # wide at 100 rows; K not a multiple of 128
     (2, 384, 19456, 1024, SWIGLU, 0, 0),    # two row tiles a wavefront, one slice
+    (2, 480, 19456, 1056, STORE, 0, 0),     # the same with an odd number of 32-row tiles: the last workgroup's upper
+    (2, 465, 19456, 1056, SWIGLU, 0, 0),    # one is past the operand
     (2, 512, 12320, 2080, ADD, 0, 2),       # two row tiles, ragged columns and K, y off 16 bytes
     (2, 260, 1056, 2048, SWIGLU, 1, 0),     # F a multiple of 16 alone, rows of h unaligned
     (8, 256, 1040, 2560, STORE, 0, 0),      # Q8_0: two slices at a time
@@ -69,6 +71,68 @@ def test_many_rows_are_the_few_rows_bits(wt, M, N, K, epi, pad, off):
         want[off + m * ldy:off + m * ldy + n * ldy] = matmul(L, wt, w, x[m:m + n], N, epi, ldy, part)
     got = matmul(L, wt, w, x, N, epi, ldy, y0, off)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def same(a, b):
+    """Equal bits where finite, and not finite in the same places."""
+    f = np.isfinite(a)
+    return np.array_equal(f, np.isfinite(b)) and np.array_equal(a[f].view(np.uint32), b[f].view(np.uint32))
+
+
+def odd_rows(r, M, K):
+    """Rows of ordinary values, and in each 32-row tile some whose values leave the formats: an infinity, a NaN, a block
+    whose fp16 scale overflows, one of subnormal scale, zeros."""
+    x = r.standard_normal((M, K)).astype(np.float32)
+    for m in range(0, M, 32):
+        for i, v in enumerate((np.inf, -np.inf, np.nan, 1e9)):
+            if m + 5 * i + 1 < M:
+                x[m + 5 * i + 1, (37 * (m + i)) % K] = v
+        x[m] *= 1e-6
+        x[min(m + 2, M - 1)] = 0
+    return x
+
+
+@pytest.mark.parametrize("wt,M,N,K,epi", [
+    (2, 256, 1008, 1152, STORE), (2, 300, 6144, 1280, ADD), (2, 480, 19456, 1056, STORE), (2, 256, 4096, 1152, SWIGLU),
+    (8, 256, 1008, 1152, STORE), (8, 300, 6144, 1280, SWIGLU),
+])
+def test_infinities_and_nans_stay_in_their_rows(wt, M, N, K, epi):
+    """Rows that hold infinities, NaN or overflowing scales are not finite where the few-row kernels' are not, and every
+    other row keeps its bits."""
+    L, r = S.lib(), np.random.default_rng(M + N)
+    w = U.empty((L.snk_q4_stripes_bytes if wt == 2 else L.snk_q8_tiles_bytes)(N, K))
+    assert (L.snk_q4_repack if wt == 2 else L.snk_q8_repack)(U.ptr(U.dev(weights(r, N, K, wt))), N, K, U.ptr(w), U.stream()) == 0
+    x = odd_rows(r, M, K)
+    cols = N // 2 if epi == SWIGLU else N
+    y0 = r.standard_normal((M, cols)).astype(np.float32)
+    got = matmul(L, wt, w, x, N, epi, cols, y0)
+    for m in range(0, M, 16):
+        want = matmul(L, wt, w, x[m:m + 16], N, epi, cols, y0[m:m + 16])
+        assert same(got[m:m + 16], want), m
+
+
+@pytest.mark.parametrize("M,K,norm", [(192, 2560, False), (640, 2560, True), (336, 5120, True)])
+def test_operand_of_infinities_and_nans(M, K, norm):
+    """The activation quantizer's tile form over such rows: the row kernel's operand, bit for bit (a NaN as a NaN)."""
+    L, r = S.lib(), np.random.default_rng(M)
+    x, nw = odd_rows(r, M, K), U.dev((1 + 0.1 * r.standard_normal(K)).astype(np.float32))
+
+    def operand(rows):
+        xa = U.empty(L.snk_xa_bytes(len(rows), K))
+        assert L.snk_quant_act(U.ptr(U.dev(rows)), len(rows), K, K, U.ptr(nw) if norm else None, 1e-6, U.ptr(xa),
+                               U.stream()) == 0
+        rec = U.host(xa, np.uint8)[:L.snk_xa_bytes(len(rows), K)].reshape(-1, 4864)
+        q = rec[:, :4096].copy().view(np.uint16)
+        k = rec[:, 4096:].copy().view(np.uint32)
+        q[np.isnan(q.view(np.float16))], k[np.isnan(k.view(np.float32))] = 0x7e00, 0x7fc00000
+        return q, k
+
+    q, k = operand(x)
+    n = L.snk_xa_bytes(32, K) // 2 // 4864  # a row tile's records
+    for m in range(0, M, 16):
+        wq, wk = operand(x[m:m + 16])
+        t = slice(m // 16 * n, (m // 16 + 1) * n)
+        assert np.array_equal(q[t], wq[:n]) and np.array_equal(k[t], wk[:n]), m
 
 
 @pytest.mark.parametrize("wt,N,K,M,many", [
@@ -273,3 +337,28 @@ def test_gate_up_of_a_wide_model_up_to_32_rows(tmp_path):
             want = got if want is None else want
             assert np.array_equal(got, want), step
     assert launches[24] == launches[32] == launches[33] + 1, launches
+
+
+def test_operand_of_chosen_rows_and_its_normed_rows(tmp_path):
+    """The activation quantizer's tile form behind a row list (the LM head's rows of a step) and with the normed rows
+    kept (the guess head's input): 800 rows of 400 sequences in one step, 400 of them sampled, against the same in steps
+    of 32 rows: logits, and the cells of the model and of its guess head."""
+    path = str(tmp_path / "m.gguf")
+    S.write_model(path, S.model_cfg(1, 4096, 8, 2, 512, 1000, nextn=1), 5)
+    n = 400
+    tok = np.random.default_rng(3).integers(0, 1000, (n, 2)).astype(np.int32)
+    res = []
+    for step in (n, 16):
+        with S.Engine(path, slots=n, ctx=64, max_rows=2 * n) as eng:
+            assert eng.guess_on(True)
+            lg = []
+            for s in range(0, n, step):
+                seq = np.repeat(np.arange(s, s + step, dtype=np.int32), 2)
+                at = 2 * np.arange(step, dtype=np.int32) + (np.arange(s, s + step) % 3 > 0)
+                eng.step(tok[s:s + step].reshape(-1), seq, np.tile(np.arange(2, dtype=np.int32), step),
+                         at.astype(np.int32), n_write=0)
+                lg.append(eng.logits(np.arange(step)).copy())
+            res.append((np.concatenate(lg), [eng.kv_save(s, 2).copy() for s in (0, 1, 17, 160, n - 1)]))
+    assert np.array_equal(res[0][0].view(np.uint32), res[1][0].view(np.uint32))
+    for a, b in zip(res[0][1], res[1][1]):
+        assert np.array_equal(a, b)

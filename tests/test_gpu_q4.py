@@ -159,7 +159,7 @@ def test_row_invariance_bitwise():
     r = np.random.default_rng(4)
     N, K = 1536, 2560
     Wq = O.quantize_q4_0(r.normal(0, 0.02, (N, K)).astype(np.float32))
-    # 300 rows: every matrix takes its row tiles in pairs (prompt rows); the 1..40-row subsets single tiles here
+    # 300 rows: the many-row kernel's 32 x 32 tiles; the 1..40-row subsets the streaming kernel's split launches
     X = r.normal(0, 1, (300, K)).astype(np.float32)
     L = S.lib()
     wbuf = U.empty(L.snk_q4_stripes_bytes(N, K))
@@ -172,8 +172,8 @@ def test_row_invariance_bitwise():
 
 @pytest.mark.parametrize("N,K", [(6144, 2560), (19456, 2560), (2560, 9728)])
 def test_row_invariance_prompt_shapes(N, K):
-    """The Qwen3-4B layer matrices (q|k|v, gate|up, down) at 300 prompt rows, where one workgroup walks every k-slice
-    of its tiles and adds them in slice order itself, against decode-sized subsets of the same rows, which the split
+    """The Qwen3-4B layer matrices (q|k|v, gate|up, down) at 300 prompt rows, where the many-row kernel walks every
+    k-slice of its tiles and adds them in slice order itself, against decode-sized subsets of the same rows, which the split
     launches and the consumer's slice sum serve: every row bit for bit the same (sn.h:1-3)."""
     r = np.random.default_rng(N + K)
     Wq = O.quantize_q4_0(r.normal(0, 0.02, (N, K)).astype(np.float32))
@@ -189,13 +189,19 @@ def test_row_invariance_prompt_shapes(N, K):
     assert np.all(np.abs(full[:4] - ref) <= ATOL + RTOL * np.abs(ref))
 
 
-def test_prompt_gate_up_swiglu_epilogue():
+@pytest.mark.parametrize("F,K,M", [
+    (3072, 2560, 256),  # two k-slices at a time
+    (3072, 2560, 300),  # one 32-row tile a wavefront
+    (9728, 1152, 512),  # two 32-row tiles a wavefront; a last slice of one group
+    (9728, 1152, 480),  # an odd number of 32-row tiles: the last workgroup's upper one is past the operand
+    (9728, 1152, 465),
+])
+def test_prompt_gate_up_swiglu_epilogue(F, K, M):
     """Prompt rows of an interleaved gate|up matrix with the SwiGLU + Q8_0 as the matmul's epilogue
-    (snk_q4_gemm_swiglu): the fp32 rows and the down projection's operand are bit for bit the matmul with its SwiGLU
-    output (snk_q4_gemm, epilogue 2) and the activation quantizer over those rows (snk_quant_act); below 256 rows the
-    call declines (1) and launches nothing."""
+    (snk_q4_gemm_swiglu), in each of its launches: the fp32 rows and the down projection's operand are bit for bit those
+    of calls of 16 rows, which the split launches, the slice sum's SwiGLU (snk_q4_gemm, epilogue 2) and the activation
+    quantizer's row kernel (snk_quant_act) serve; below 256 rows the call declines (1) and launches nothing."""
     r = np.random.default_rng(12)
-    F, K, M = 3072, 2560, 300
     N = 2 * F
     Wq = O.quantize_q4_0(r.normal(0, 0.02, (N, K)).astype(np.float32))
     X = r.normal(0, 1, (M, K)).astype(np.float32)
@@ -203,16 +209,20 @@ def test_prompt_gate_up_swiglu_epilogue():
     st = U.stream()
     wbuf = U.empty(L.snk_q4_stripes_bytes(N, K))
     assert L.snk_q4_repack(U.ptr(U.dev(Wq)), N, K, U.ptr(wbuf), st) == 0
-    Y, xa = gemm_gpu(None, N, K, X, epi=2, wbuf=wbuf)  # silu(gate) * up through the split-free launch and reduction
-    dxa = U.dev(xa)
+    dxa = U.dev(np.zeros(L.snk_xa_bytes(M, K), np.uint8))
+    assert L.snk_quant_act(U.ptr(U.dev(X)), M, K, K, None, 0.0, U.ptr(dxa), st) == 0
     h = U.dev(np.zeros((M, F), np.float32))
     xo = U.dev(np.zeros(L.snk_xa_bytes(M, F), np.uint8))
     assert L.snk_q4_gemm_swiglu(U.ptr(wbuf), U.ptr(dxa), M, N, K, U.ptr(h), U.ptr(xo), st) == 0
     gh = U.host(h, np.float32)[:M * F].reshape(M, F)
-    assert np.array_equal(gh.view(np.uint32), Y.view(np.uint32))
-    ref_xo = U.dev(np.zeros(L.snk_xa_bytes(M, F), np.uint8))
-    assert L.snk_quant_act(U.ptr(U.dev(Y)), M, F, F, None, 0.0, U.ptr(ref_xo), st) == 0
-    assert np.array_equal(U.host(xo, np.uint8), U.host(ref_xo, np.uint8))
+    tile = L.snk_xa_bytes(32, F) // 2  # a 16-row tile's records
+    go = U.host(xo, np.uint8)[:L.snk_xa_bytes(M, F)].reshape(-1, tile)
+    for m in range(0, M, 16):
+        Y, _ = gemm_gpu(None, N, K, X[m:m + 16], epi=2, wbuf=wbuf)
+        assert np.array_equal(gh[m:m + 16].view(np.uint32), Y.view(np.uint32)), m
+        ref = U.dev(np.zeros(L.snk_xa_bytes(len(Y), F), np.uint8))
+        assert L.snk_quant_act(U.ptr(U.dev(Y)), len(Y), F, F, None, 0.0, U.ptr(ref), st) == 0
+        assert np.array_equal(go[m // 16], U.host(ref, np.uint8)[:tile]), m
     assert L.snk_q4_gemm_swiglu(U.ptr(wbuf), U.ptr(dxa), 200, N, K, U.ptr(h), U.ptr(xo), st) == 1
 
 

@@ -94,7 +94,7 @@ def test_q8_epilogues_and_row_invariance():
     for i in (0, 16, 32):  # each row alone equals its row in the 33-row matmul, bit for bit
         Yi, _ = gemm_q8(Wq, N, K, X[i:i + 1], wbuf=wbuf)
         assert np.array_equal(Yi[0].view(np.uint32), Y[i].view(np.uint32))
-    # 280 rows (row tiles in pairs, from other offsets) hold the same 33 rows' results
+    # 280 rows (the many-row kernel, from other offsets) hold the same 33 rows' results
     Xl = np.concatenate([r.normal(0, 1, (200, K)).astype(np.float32), X, X[:47]])
     Yl, _ = gemm_q8(Wq, N, K, Xl, wbuf=wbuf)
     assert np.array_equal(Yl[200:233].view(np.uint32), Y.view(np.uint32))
