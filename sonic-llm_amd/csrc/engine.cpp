@@ -925,8 +925,8 @@ struct Dev {
             return ks < 0 ? -1 : 0;
         });
     }
-    // prompt rows: gate|up with its SwiGLU + Q8_0 as the epilogue (the rows h and the down projection's operand in
-    // xa2); false when the shape does not take it
+    // many rows: gate|up with its SwiGLU + Q8_0 as the many-row kernel's epilogue (the rows h and the down projection's
+    // operand in xa2); false when the shape does not take it
     bool gemm_swiglu(const uint8_t* w, int M) {
         const int F = e->F, E = e->E;
         if (!e->xa2 || !q4_gemm_swiglu_fits(M, 2 * F, E, e->wt)) return false;

@@ -1064,8 +1064,9 @@ typedef float floatx32 __attribute__((ext_vector_type(32)));
 // in slice order. With WK > 1 a round of WK slices ends with the parts past the first handing their sums to the first
 // through LDS, which adds them one by one.
 //
-// What bounds it: per block and tile the MFMAs take 96 cycles and the wavefront's other 29 instructions 90, and the two
-// overlap little on this SIMD (32 MFMAs + 32 fmas took the sum of their times with 2 wavefronts a SIMD).
+// What bounds it: the MFMAs and the vector work beside them, which hardly overlap. 512 rows of 19456 x 2560 (counters): a
+// block and tile takes 257 cycles of a SIMD, 96 of them with the matrix core busy and 153 with one of its 36 vector
+// instructions issuing.
 //
 // Grid: 1-D, linear id L on XCD L mod 8. The XCDs are xm groups along the rows times 8 / xm along the columns, so that
 // an XCD's L2 holds its share of the activation: mx row tiles a group, interleaved.
@@ -1417,7 +1418,8 @@ __global__ __launch_bounds__(256) void k_q4_reduce(GemmArgs a) {
 // the consumer one more partial sum to read.
 #define Q4_WIDE (8 * 768)  // stripes of an LM-head-wide matrix
 #define Q4_MANY_ROWS 256   // rows from which every matrix takes the many-row kernel
-// 32 x 32 tiles (of rows, padding not counted) from which fewer rows' gate|up takes it with its SwiGLU (q4_gemm_swiglu_fits)
+// 32 x 32 tiles (of rows, padding not counted) from which fewer rows' gate|up takes it with its SwiGLU
+// (q4_gemm_swiglu_fits)
 #define SWIGLU_WIDE_TILES 1200
 GemmPlan q4_plan(int N, int K, int wt) {
     GemmPlan p;
@@ -2013,8 +2015,11 @@ static void launch_resid(int km, int nt, float* x, const float* part, int ks, in
 int resid_quant(float* x, const float* part, int ks, int M, int K, const float* nw, float eps, uint8_t* xa,
                 hipStream_t st, bool add, float* xn, const uint8_t* next_w, int next_N, int next_K, int wt) {
     if (M <= 0) return 0;
-    // (next_w: the next matmul's first groups into the Infinity Cache by extra workgroups; decode-sized rows only,
-    // where that matmul streams its slices)
+    // (next_w: the next matmul's first groups into the Infinity Cache by extra workgroups, below 256 rows. They are the
+    // first of each k-slice, what the streaming kernel's workgroups load first; the many-row kernel walks the slices in
+    // turn and still finds them there. A 6-layer step whose gate|up is that kernel's, with / without, us: 2560 wide, 64
+    // rows 565 / 573, 128 725 / 735, 192 933 / 936, 224 1050 / 1043, 255 1130 / 1120; 1024 wide, 192 rows 494 / 509,
+    // 255 503 / 520)
     WeightPrefetch pf{};
     int npf = 0;
     if (next_w && M < Q4_MANY_ROWS) {

@@ -115,13 +115,12 @@ __global__ __launch_bounds__(64) void k_q6k_dequant(const uint8_t* __restrict__ 
 // grid (rows M), a wavefront a block of the row (4 to 16): row m (source rows[m] of X when given) RMS-normed by nw when
 // given (scale 1/sqrt(mean x^2 + eps), summed by the first 256 threads as the activation quantizer does: thread t over
 // elements t, t + 256, ..), then each wavefront quantizes its block (and those 16 on) with lane l holding elements
-// 4 l .. 4 l + 3 (32 rows of 2560: 4.1 us; 4 wavefronts a row that loaded
-// after the sum: 6.8): ggml quantize_row_q8_K_ref (max = the
-// value of largest |x|, the first on ties; iscale = -127 / max; q = min(127, round-half-even(iscale * x)); d =
-// 1 / iscale; an all-zero block: d = 0, q = 0).
+// 4 l .. 4 l + 3 (32 rows of 2560: 4.1 us; 4 wavefronts a row that loaded after the sum: 6.8): ggml
+// quantize_row_q8_K_ref (max = the value of largest |x|, the first on ties; iscale = -127 / max; q = min(127,
+// round-half-even(iscale * x)); d = 1 / iscale; an all-zero block: d = 0, q = 0).
 __global__ __launch_bounds__(1024) void k_quant_q8k(const float* __restrict__ X, const int32_t* __restrict__ rows,
-                                                   int K, int ldx, const float* __restrict__ nw, float eps,
-                                                   uint8_t* __restrict__ xk) {
+                                                    int K, int ldx, const float* __restrict__ nw, float eps,
+                                                    uint8_t* __restrict__ xk) {
     __shared__ float red_s[4];
     const int m = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6, nwv = blockDim.x >> 6, nb = K / 256;
     const float* x = X + (size_t) (rows ? rows[m] : m) * ldx;
@@ -305,7 +304,9 @@ void q6k_dequant(const uint8_t* tiles, int N, int K, float* out, hipStream_t st)
 }
 void quant_q8k(const float* x, const int32_t* rows, int M, int K, int ldx, const float* nw, float eps, uint8_t* xk,
                hipStream_t st) {
-    if (M > 0) hipLaunchKernelGGL(k_quant_q8k, dim3(M), dim3(64 * (K / 256 < 4 ? 4 : K / 256 > 16 ? 16 : K / 256)), 0, st, x, rows, K, ldx, nw, eps, xk);
+    if (M <= 0) return;
+    const int waves = K / 256 < 4 ? 4 : K / 256 > 16 ? 16 : K / 256;
+    hipLaunchKernelGGL(k_quant_q8k, dim3(M), dim3(64 * waves), 0, st, x, rows, K, ldx, nw, eps, xk);
 }
 int q6k_gemm(const uint8_t* tiles, const uint8_t* xk, int M, int N, int K, float* y, int ldy, hipStream_t st) {
     if (M <= 0) return 0;

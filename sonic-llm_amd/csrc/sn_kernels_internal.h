@@ -67,8 +67,8 @@ static inline int fe_slice_index(int ks) {
 
 // Launch shape of one matrix: a workgroup owns 4 spw stripes (a "set": spw per wavefront) and gps consecutive 4-block
 // groups (a slice). Layer-sized matrices at decode row counts run the streaming kernel (sspw stripes a wavefront,
-// smt row tiles a workgroup); LM-head-wide matrices and prompt-sized row counts the ring kernel (spw, sets). The
-// slices are the same for both, so a row's sums do not depend on the kernel.
+// smt row tiles a workgroup); LM-head-wide matrices the ring kernel (spw, sets), many rows the many-row kernel
+// (wide_takes). The slices are the same for all, so a row's sums do not depend on the kernel.
 struct GemmPlan {
     int nstripes, ngroups, spw, sets, ks, gps;
     bool stream;    // the streaming kernel serves this matrix below the many-row kernel's rows
@@ -81,9 +81,10 @@ GemmPlan q4_plan(int N, int K, int wt = WT_Q4_0);
 // the raw matmul with an explicit plan (tuning): mt row tiles a workgroup, spw stripes a wavefront, G groups a slice
 // loaded at once (G 0: the default plan); the slice count, or -1
 // part[ks][M][N] added in slice order into y [M][N]
-// The gate|up matmul of many rows with its SwiGLU: from 256 rows, or fewer where their tiles fill the chip, a Q4_0
-// stripe-interleaved matrix of N = 2F (F a multiple of 128) through the many-row kernel (k_q4_gemm_w) with silu(gate) * up written as fp32 rows h [M][F] and
-// as the Q8_0 operand xo (K = F), the same bits as the matmul's slices through k_swiglu_quant. xo must not be xa.
+// The gate|up matmul of many rows with its SwiGLU: from 256 rows, or fewer (33 and more) where their tiles fill the
+// chip, a Q4_0 stripe-interleaved matrix of N = 2F (F a multiple of 128) through the many-row kernel (k_q4_gemm_w) with
+// silu(gate) * up written as fp32 rows h [M][F] and as the Q8_0 operand xo (K = F), the same bits as the matmul's
+// slices through k_swiglu_quant. xo must not be xa.
 // Returns 1, or 0 when the shape does not qualify (nothing launched: use the matmul and swiglu_quant).
 int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, float* h, uint8_t* xo, hipStream_t st,
                    int wt);

@@ -433,8 +433,9 @@ def test_attention_list_forms_give_the_same_steps(tiny):
 def test_prompt_chunking_does_not_change_the_next_row(tmp_path):
     """A prompt fed in one step or in several gives the same cells and so the same next row, bit for bit (qbench.m's
     read_chunks, qbench.m:124-130): 600 prompt rows in one step (the many-row matmul and run items at 600 rows),
-    in 200-row steps (q|k|v with its RoPE epilogue, the down projection split, chunk items), and in 64 + 536 (a step of
-    decode-sized launches before one of many rows), then the same decode row. The model's
+    in 200-row steps (q|k|v with its RoPE epilogue, the down projection split, chunk items), in 64 + 536 (a step of
+    decode-sized launches before one of many rows), and in 150-row steps without the epilogues (the workgroup-per-row
+    QK-RoPE adding the k-slice sums), then the same decode row. The model's
     matrices all split K (n_embd 1024: 2 slices) and its gate|up is wide enough (n_ff 3072: 384 stripes) for the prompt
     SwiGLU epilogue."""
     path = str(tmp_path / "w.gguf")
@@ -444,8 +445,10 @@ def test_prompt_chunking_does_not_change_the_next_row(tmp_path):
     toks = r.integers(0, 1000, 600).astype(np.int32)
     nxt = np.array([int(r.integers(0, 1000))], np.int32)
     outs = []
-    for cuts in ([0, 600], [0, 200, 400, 600], [0, 64, 600]):
+    for cuts in ([0, 600], [0, 200, 400, 600], [0, 64, 600], [0, 150, 300, 450, 600]):
         with S.Engine(path, slots=1, ctx=1024, max_rows=600) as eng:
+            if cuts[1] == 150:
+                eng.fuse(False)
             for a, b in zip(cuts[:-1], cuts[1:]):
                 eng.step(toks[a:b], np.zeros(b - a, np.int32), np.arange(a, b, dtype=np.int32),
                          np.array([b - a - 1], np.int32), n_write=0)
