@@ -1245,14 +1245,18 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(OC
     if (wk > 0 || col >= a.N) return;
     float* o = a.y + (size_t) row0 * a.ldy + col;
     const int nr = a.M - row0;
-    for (int mt = 0; mt < MT; ++mt)
-        for (int v = 0; v < 16; ++v) {
-            const int rr = 32 * mt + 8 * (v / 4) + 4 * eh + v % 4;
-            if (rr < nr) {
-                if (a.epi == EPI_ADD) o[(size_t) rr * a.ldy] += tot[mt][v];
-                else o[(size_t) rr * a.ldy] = tot[mt][v];
-            }
+    for (int mt = 0; mt < MT; ++mt) {
+        auto row = [&](int v) { return 32 * mt + 8 * (v / 4) + 4 * eh + v % 4; };
+        // (added: every load before the first add and store, rows past M clamped; a load and a wait for each row, 256 rows
+        // of 1000 x 1056 took 10.3 us, so 7.3, 512 of 2560 x 4096 27.7, so 24.0)
+        if (a.epi == EPI_ADD) {
+            float y[16];
+            for (int v = 0; v < 16; ++v) y[v] = o[(size_t) min(row(v), nr - 1) * a.ldy];
+            for (int v = 0; v < 16; ++v) tot[mt][v] = y[v] + tot[mt][v];
         }
+        for (int v = 0; v < 16; ++v)
+            if (row(v) < nr) o[(size_t) row(v) * a.ldy] = tot[mt][v];
+    }
 }
 
 // The few-row matmul (M <= 4 rows: the reference's mat-vec rows, mv_q4, kernels.metal:1324-1411). One lane per output

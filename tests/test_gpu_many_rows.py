@@ -184,18 +184,12 @@ def test_operand_of_many_rows_is_the_row_kernels(M, K, norm):
         assert np.array_equal(q[m:m + 16], wq) and np.array_equal(d[m:m + 16].view(np.uint32), wd.view(np.uint32))
 
 
-def test_operand_of_ragged_rows_costs_what_whole_tiles_do():
-    """A row tile's workgroups share its rows in one L2 whatever the number of tiles: 520 rows of 4096 with the norm (33
-    tiles) take about the time of 512 (32), not that of every XCD reading every row (1.8 times). Times of 20 calls as one
-    graph, the least of 12 replays in turn."""
-    L, K = S.lib(), 4096
-    nw = torch.ones(K, device="cuda")
-    graphs, keep = [], []
-    for M in (512, 520):
-        x, xa = torch.randn(M, K, device="cuda"), U.empty(L.snk_xa_bytes(M, K))
+def least_us(calls):
+    """The device time of each call: 20 of it as one graph, the least of 12 replays in turn."""
+    graphs = []
+    for call in calls:
         s = torch.cuda.Stream()
         with torch.cuda.stream(s):
-            call = lambda: L.snk_quant_act(U.ptr(x), M, K, K, U.ptr(nw), 1e-6, U.ptr(xa), U.stream())
             assert call() == 0
             s.synchronize()
             g = torch.cuda.CUDAGraph()
@@ -203,8 +197,7 @@ def test_operand_of_ragged_rows_costs_what_whole_tiles_do():
                 for _ in range(20):
                     assert call() == 0
         graphs.append(g)
-        keep.append((x, xa))
-    best = [float("inf")] * 2
+    best = [float("inf")] * len(graphs)
     for _ in range(12):
         for i, g in enumerate(graphs):
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -212,9 +205,34 @@ def test_operand_of_ragged_rows_costs_what_whole_tiles_do():
             g.replay()
             b.record()
             torch.cuda.synchronize()
-            best[i] = min(best[i], a.elapsed_time(b))
-    print("512 rows %.2f us, 520 rows %.2f us" % tuple(50 * t for t in best))
-    assert best[1] < 1.45 * best[0]
+            best[i] = min(best[i], 50 * a.elapsed_time(b))
+    print(" ".join("%.2f us" % t for t in best))
+    return best
+
+
+def test_operand_of_ragged_rows_costs_what_whole_tiles_do():
+    """A row tile's workgroups share its rows in one L2 whatever the number of tiles: 520 rows of 4096 with the norm (33
+    tiles) take about the time of 512 (32), not that of every XCD reading every row (1.8 times)."""
+    L, K = S.lib(), 4096
+    nw, keep, calls = torch.ones(K, device="cuda"), [], []
+    for M in (512, 520):
+        x, xa = torch.randn(M, K, device="cuda"), U.empty(L.snk_xa_bytes(M, K))
+        keep.append((x, xa))
+        calls.append(lambda x=x, xa=xa, M=M: L.snk_quant_act(U.ptr(x), M, K, K, U.ptr(nw), 1e-6, U.ptr(xa), U.stream()))
+    whole, ragged = least_us(calls)
+    assert ragged < 1.45 * whole
+
+
+def test_added_output_costs_little_more_than_a_stored_one():
+    """The many-row kernel's add epilogue loads a tile's output before it stores any of it: 256 rows of 1000 x 1056 added
+    take about the time of the same stored, not a load's wait for each of a lane's 16 rows (1.5 times)."""
+    L, M, N, K = S.lib(), 256, 1000, 1056
+    w, xa, y = U.empty(L.snk_q4_stripes_bytes(N, K)), U.empty(L.snk_xa_bytes(M, K)), U.empty(4 * M * N)
+    nb = L.snk_q4_workspace_bytes(M, N, K)
+    ws = U.empty(nb)
+    store, add = least_us([lambda e=e: L.snk_q4_gemm(U.ptr(w), U.ptr(xa), M, N, K, U.ptr(y), N, e, U.ptr(ws), nb, U.stream())
+                           for e in (STORE, ADD)])
+    assert add < 1.3 * store
 
 
 @pytest.mark.parametrize("M,N,K,epi,pad,off", [
