@@ -1526,13 +1526,15 @@ static bool launch_gemv(const GemmPlan& p, const GemmArgs& a, hipStream_t st) {
 // - from 96 rows with T = 2048 tiles of 32 x 32 on: 19456 x 2560 at 100 rows (T = 2432) 36.2 / 26.6 (49.6 / 28.7);
 //   12288 x 2048 at 192 (2304) 35.9 / 22.4 (48.3 / 24.4). (Smaller launches gain too, 5120 x 2048 at 96 rows 13.1 / 8.8 and 6144 x
 //   2560 at 96 16.1 / 14.8, but not all: 2560 x 4096 at 96 rows 11.9 / 14.1. Not taken.)
-// - from 192 rows with at most 32 groups, where the rows times the column tiles times the groups outweigh the walk:
-//   the wide kernel's time is its walk of w groups one after another while its tiles fit the chip at once,
-//   the streaming kernel's grows with the tiles times the groups. Sides of the line at (N x K, rows): 256 x 4096, 255
-//   6.8 / 13.6 (7.0 / 14.6); 1024 x 1536, 224 7.8 / 8.7 (8.0 / 9.1); 1024 x 2048, 192 8.1 / 8.6, and 224 8.8 / 8.7
-//   (9.3 / 9.1); 1024 x 3072, 224 10.9 / 11.4 (12.0 / 12.0); 1536 x 4096, 208 13.0 / 13.8, and 224 14.4 / 13.8 (15.1 /
-//   15.0); 512 x 1024, 224 5.9 / 5.9, 768 x 1024, 192 6.4 / 5.9; 2560 x 4096, 192 17.5 / 14.3 (18.2 / 15.3). Deeper ones
-//   not: 2560 x 9728 at 224 rows 31.6 / 38.0, Q8_0 43.2 / 40.6.
+// - from 192 rows with at most 32 groups, where the rows times the column tiles times the slices' groups outweigh the
+//   walk: the wide kernel's time is its walk of w groups one after another while its tiles fit the chip at once, the
+//   streaming kernel's grows with the tiles times the groups (a short last slice counts whole: its launch and its sum
+//   cost the same). Sides of the line at (N x K, rows): 256 x 4096, 255 6.8 / 13.6 (7.0 / 14.6); 512 x 1056, 224 6.5 /
+//   6.5; 768 x 1184, 224 6.8 / 7.2, and 240 7.2 / 7.2; 1024 x 1536, 224 7.8 / 8.7 (8.0 / 9.1); 1000 x 1600, 192 8.1 /
+//   8.5, and 208 8.8 / 8.5; 1024 x 2048, 192 8.1 / 8.6, and 224 8.8 / 8.7 (9.3 / 9.1); 1000 x 2080, 192 8.7 / 9.2, and
+//   224 10.8 / 9.3; 1024 x 3072, 224 10.9 / 11.4 (12.0 / 12.0); 1536 x 4096, 208 13.0 / 13.8, and 224 14.4 / 13.8 (15.1
+//   / 15.0); 768 x 1024, 192 6.4 / 5.9; 2560 x 4096, 192 17.5 / 14.3 (18.2 / 15.3). Deeper ones not: 2560 x 9728 at
+//   224 rows 31.6 / 38.0, Q8_0 43.2 / 40.6.
 static bool wide_takes(int M, const GemmPlan& p) {
     const long nt = (p.nstripes + 1) / 2, T = (M + 31) / 32 * nt;
     if (M >= Q4_MANY_ROWS || (M >= 96 && T >= 2048)) return true;
@@ -1540,7 +1542,7 @@ static bool wide_takes(int M, const GemmPlan& p) {
     // the groups walked: with two slices at a time, twice the longer part's (an odd last slice leaves one part idle)
     const int rounds = (p.ks + 1) / 2, last = p.ngroups - (rounds - 1) * 2 * p.gps;
     const long w = p.ks == 1 ? p.ngroups : 2 * ((rounds - 1) * p.gps + std::min(p.gps, last));
-    return M * nt * p.ngroups >= 32 * w * (8 * w + 80);
+    return M * nt * p.ks * p.gps >= 32 * w * (8 * w + 80);
 }
 static GemmArgs wide_args(const uint8_t* w, const uint8_t* xa, int M, int N, int K, const GemmPlan& p) {
     GemmArgs a{};

@@ -139,6 +139,7 @@ def test_operand_of_infinities_and_nans(M, K, norm):
     (2, 256, 4096, 255, False), (8, 256, 4096, 200, False),   # narrow and deep: few tiles, a long walk
     (2, 1024, 3072, 255, False), (2, 1024, 1536, 224, False), (8, 768, 3072, 240, False),
     (2, 1024, 2048, 207, False), (2, 1024, 2048, 208, True),  # the line
+    (8, 1000, 2080, 201, False), (2, 1000, 2080, 202, True),  # a short last slice counts whole
     (2, 768, 1024, 191, False), (2, 768, 1024, 192, True), (2, 256, 4096, 256, True),
     (2, 2560, 4096, 192, True), (8, 6144, 2560, 200, True),
 ])
