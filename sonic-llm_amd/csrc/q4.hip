@@ -1883,7 +1883,9 @@ int q4_gemm_swiglu(const uint8_t* w, const uint8_t* xa, int M, int N, int K, flo
 }
 
 // 4 columns a thread where the slices' and the output's rows are 16-byte aligned. Up to 256 workgroups' worth of
-// threads go as single wavefronts, so that a few rows still reach every CU.
+// threads go as single wavefronts, so that a few rows still reach every CU. (Two slices as two: the clamped loads of
+// four made SwiGLU's sum slower than one at a time, 6144 x 1024 at 48 rows with the matmul 8.6 us, 8.95, so 8.8; three
+// as four, and the scalar form, measured the same.)
 static void launch_reduce(const GemmArgs& a, hipStream_t st) {
     const int cols = a.epi == EPI_SWIGLU ? a.N / 2 : a.N;
     const bool v4 = a.N % 4 == 0 && a.ldy % 4 == 0 && ((uintptr_t) a.part | (uintptr_t) a.y) % 16 == 0;
@@ -1892,6 +1894,7 @@ static void launch_reduce(const GemmArgs& a, hipStream_t st) {
     const dim3 grid((unsigned) ((n + wg - 1) / wg)), block(wg);
     if (v4) {
         if (a.ks == 1) hipLaunchKernelGGL((k_q4_reduce<4, 1>), grid, block, 0, st, a);
+        else if (a.ks == 2) hipLaunchKernelGGL((k_q4_reduce<4, 2>), grid, block, 0, st, a);
         else if (a.ks <= 4) hipLaunchKernelGGL((k_q4_reduce<4, 4>), grid, block, 0, st, a);
         else hipLaunchKernelGGL((k_q4_reduce<4, 8>), grid, block, 0, st, a);
     } else {

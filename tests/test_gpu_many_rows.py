@@ -238,6 +238,7 @@ def test_added_output_costs_little_more_than_a_stored_one():
 
 @pytest.mark.parametrize("M,N,K,epi,pad,off", [
     (1, 64, 32, STORE, 0, 0),          # one slice
+    (33, 2080, 1024, SWIGLU, 0, 0),    # two slices
     (3, 4, 4096, ADD, 0, 0),           # one thread a row
     (5, 1001, 4096, STORE, 0, 0),      # columns not a multiple of 4: the scalar form
     (7, 1000, 4096, ADD, 3, 0),        # rows of y unaligned: the scalar form
