@@ -304,8 +304,8 @@ __global__ __launch_bounds__(256) void k_argmax_part(const float* __restrict__ l
             }
         }
     };
-    // (a branch around the whole scan: around each id's 8 compares 32 banned rows of 151936 took 11.4 us, so 8.5, and without
-    // bans 9.3, so 6.7)
+    // (a branch around the whole scan: around each id's 8 compares 32 banned rows of 151936 took 11.4 us, so 8.5, and
+    // without bans 9.3, so 6.7)
     if (nb > 0) scan(std::true_type{});
     else scan(std::false_type{});
     if (LSE && p.tp.m1 > -INFINITY)

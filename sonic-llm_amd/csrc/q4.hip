@@ -1524,8 +1524,8 @@ static bool launch_gemv(const GemmPlan& p, const GemmArgs& a, hipStream_t st) {
 // the other kernels' slices cost more than the wide tiles leave idle. us on MI355X of the streaming kernel with its
 // slice sum / this one, Q4_0 (Q8_0 in brackets):
 // - from 96 rows with T = 2048 tiles of 32 x 32 on: 19456 x 2560 at 100 rows (T = 2432) 36.2 / 26.6 (49.6 / 28.7);
-//   12288 x 2048 at 192 (2304) 35.9 / 22.4 (48.3 / 24.4). (Smaller launches gain too, 5120 x 2048 at 96 rows 13.1 / 8.8 and 6144 x
-//   2560 at 96 16.1 / 14.8, but not all: 2560 x 4096 at 96 rows 11.9 / 14.1. Not taken.)
+//   12288 x 2048 at 192 (2304) 35.9 / 22.4 (48.3 / 24.4). (Smaller launches gain too, 5120 x 2048 at 96 rows 13.1 / 8.8
+//   and 6144 x 2560 at 96 16.1 / 14.8, but not all: 2560 x 4096 at 96 rows 11.9 / 14.1. Not taken.)
 // - from 192 rows with at most 32 groups, where the rows times the column tiles times the slices' groups outweigh the
 //   walk: the wide kernel's time is its walk of w groups one after another while its tiles fit the chip at once, the
 //   streaming kernel's grows with the tiles times the groups (a short last slice counts whole: its launch and its sum
@@ -1577,7 +1577,8 @@ static void launch_wide(int wt, bool sw, const GemmPlan& p, GemmArgs& a, hipStre
         else sw ? launch_w<WT_Q8_0, 1, 4, 1, 3, true>(p, a, st) : launch_w<WT_Q8_0, 1, 4, 1, 3, false>(p, a, st);
     } else {
         if (cfg == 2) sw ? launch_w<WT_Q4_0, 1, 2, 2, 3, true>(p, a, st) : launch_w<WT_Q4_0, 1, 2, 2, 3, false>(p, a, st);
-        else if (cfg == 1) sw ? launch_w<WT_Q4_0, 1, 4, 1, 3, true>(p, a, st) : launch_w<WT_Q4_0, 1, 4, 1, 3, false>(p, a, st);
+        else if (cfg == 1) sw ? launch_w<WT_Q4_0, 1, 4, 1, 3, true>(p, a, st)
+                              : launch_w<WT_Q4_0, 1, 4, 1, 3, false>(p, a, st);
         else sw ? launch_w<WT_Q4_0, 2, 4, 1, 3, true>(p, a, st) : launch_w<WT_Q4_0, 2, 4, 1, 3, false>(p, a, st);
     }
 }
